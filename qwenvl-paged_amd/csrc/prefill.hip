@@ -4,22 +4,22 @@
 // PagedAttention.h:43-44; tests/EndToEnd.test.cpp:252-256), so every output
 // row here is the decode of its position.
 //
-// MFMA path (bf16 cache, head_dim 128, GQA group <= 16, power-of-two
-// tokens_per_block >= 16). A work item is (sequence b, kv head g, 16 new
-// positions p0 .. p0 + 15, up to 8 query heads of g's group). Its workgroup
-// streams tokens [0, p0 + 16) of kv head g in 32-token tiles: each tile is
-// loaded once, from HBM straight into LDS, one tile of compute ahead of its
+// MFMA path (bf16 or fp16 cache, head_dim 128 or 64, power-of-two
+// tokens_per_block >= 16). The rows of (sequence b, kv head g) are its new
+// positions times the G query heads of g's group, position-major, so row r is
+// head r % G at position q_start + r / G; a work item is 128 consecutive rows
+// (a cut may fall inside a position: every wave is full for any group size).
+// Its workgroup streams the tokens its last row sees in 32-token tiles: each
+// tile is loaded once, straight into LDS, one tile of compute ahead of its
 // use, into a double buffer holding the K and V rows as in the frame (16-byte
 // chunks XOR-permuted by row so the fragment reads spread over the banks; the
-// PV operands come out of V transposed by ds_read_b64_tr_b16), and every wave
-// runs the tile math of mfma_tile.h for its two query heads with the 16
-// positions in the MFMA columns, column c
-// seeing tokens t <= p0 + c (masks only on tiles that reach p0). The tile
-// loop is software-pipelined: PV of tile t runs beside QK and the softmax of
-// tile t + 1. A wave therefore covers the whole causal context of its
-// queries: no split, no merge. Items are launched longest context first so
-// the short ones fill the tail. Each K/V tile feeds 16 positions x up to 8
-// heads from LDS.
+// PV operands come out of V transposed by ds_read_b64_tr_b16). Each of the
+// four waves holds 32 of the rows in the MFMA columns, a column seeing the
+// tokens up to its position (masks only on tiles that reach the item's first
+// position). The tile loop is
+// software-pipelined over three tiles: PV of tile t - 1 and QK of tile t + 1
+// run beside the softmax of tile t. Items are launched longest context first so the short ones fill the
+// tail.
 //
 // Decode path (any other shape): one virtual sequence per new position (same
 // frames, context p + 1), packed into a private batch and run through
@@ -37,35 +37,62 @@ namespace {
 
 constexpr int kPrefillWaves = 4;
 constexpr int kPrefillThreads = kPrefillWaves * 64;
-constexpr int kPrefillPositions = 16;     // MFMA columns
-constexpr int kPrefillHeadsPerItem = 8;   // two query heads per wave
-constexpr int kHeadBytes = 256;           // 128 bf16
+constexpr int kPrefillRows = kPrefillWaves * 32;  // rows per item: the 32 MFMA columns of each wave
 // Block ids per virtual batch of the decode-kernel path.
 constexpr size_t kMaxVirtualIds = size_t{1} << 20;
 
-// One K/V tile in LDS: K and V rows as in the frame (token-major). PV MFMA n
-// takes dims 16n .. 16n + 15 as its rows; lane (c, j) needs V[4i + j][16n + c]
-// for i = 0 .. 7 (the k order of the P operand). ds_read_b64_tr_b16 hands lane
-// c of each 16-lane group element c % 4 of the 8 bytes that lane 4e + c / 4
-// of the group addressed, as element e: so lane (c, j) addresses dims
-// 16n + 4 (c % 4) .. + 3 of token 4 (c / 4 + 4h) + j, and two such reads
-// (h = 0, 1) give its eight operand elements.
-struct PrefillTile {
-    uint8_t k[kTileTokens][kHeadBytes];
-    uint8_t v[kTileTokens][kHeadBytes];
-};
-// Byte of (row, logical byte) in a swizzled 256-byte row: 16-byte chunk x at x ^ (row % 16).
-__device__ inline uint32_t swz(int row, int byte) {
-    return 16u * static_cast<uint32_t>((byte >> 4) ^ (row & 15)) + static_cast<uint32_t>(byte & 15);
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef short v4i16 __attribute__((ext_vector_type(4)));
+typedef uint32_t uint2v __attribute__((ext_vector_type(2)));
+
+// The tile math runs on 32x32x16 MFMAs, lane l = (c = l % 32, h = l / 32).
+// Beside vector work one of them takes 6 cycles less than the two 16x16x32
+// MFMAs it replaces (measured with four vector instructions per 16 cycles of
+// matrix work: 41.6 against 47.8 cycles). S^T = K Q^T: A row c is token c of
+// the tile, so score register r of lane (c, h) is token (r % 4) + 8 (r / 4) +
+// 4h for column c. O^T += V^T P^T: the eight weights r = 8ks .. 8ks + 7 of a
+// lane are the B operand of k-step ks as they are (k index 8h + e is token
+// 16ks + 8 (e / 4) + 4h + e % 4), and row c of block n is dim 32n + c.
+template <bool kF16>
+__device__ inline floatx16 mfma32(const u32x4& a, const u32x4& b, floatx16 c) {
+    if constexpr (kF16) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c,
+                                                      0, 0, 0);
+    } else {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b),
+                                                       c, 0, 0, 0);
+    }
+}
+
+// K and V tiles in LDS: rows as in the frame (token-major), K in a ring of two
+// tiles, V in a ring of three. ds_read_b64_tr_b16 hands lane i of each 16-lane
+// group element i % 4 of the 8 bytes that lane 4e + i / 4 of the group
+// addressed, as element e: with the group's lanes on tokens t .. t + 3 (by
+// i / 4) and 16 dims, lane i gets dim i of the four tokens, half of a PV
+// operand.
+constexpr int kKRing = 2;
+constexpr int kVRing = 3;
+// The LDS rows hold their 16-byte chunks XOR-permuted by row, so that the 64
+// lanes of a read spread over the banks: chunk x of row r lies at x ^ key(r).
+// K is read a chunk of 32 rows at a time, V four neighbouring chunks of eight
+// rows. (A 128-byte row covers half of the 256-byte bank period: its key has
+// three bits and row pairs share it.)
+template <int kD>
+__device__ inline int k_key(int row) {
+    return kD == 128 ? row & 15 : (row >> 1) & 7;
+}
+template <int kD>
+__device__ inline int v_key(int row) {
+    return kD == 128 ? ((row & 3) << 2) | ((row >> 2) & 3) : (((row >> 1) & 1) << 2) | ((row >> 2) & 3);
 }
 
 struct PrefillItem {
-    int32_t b;     // sequence
-    int32_t g;     // kv head
-    int32_t p0;    // first position of the block
-    int32_t np;    // positions in the block, 1 .. 16
-    int32_t row0;  // query / output row of p0
-    int32_t h0;    // first query head of the group handled by the item
+    int32_t b;      // sequence
+    int32_t g;      // kv head
+    int32_t start;  // the sequence's first new position
+    int32_t r0;     // first row of the item
+    int32_t nrows;  // rows of (b, g): new positions x G
+    int32_t row0;   // query / output row of the first new position
 };
 static_assert(sizeof(PrefillItem) == 6 * sizeof(int32_t), "PrefillItem is six int32");
 
@@ -74,258 +101,441 @@ __device__ inline const __attribute__((address_space(4))) T* as_const(const T* p
     return (const __attribute__((address_space(4))) T*)(ptr);
 }
 
-__device__ inline u32x4 lds16(const uint8_t* p) { return *reinterpret_cast<const u32x4*>(p); }
-typedef short v4i16 __attribute__((ext_vector_type(4)));
-typedef uint32_t uint2v __attribute__((ext_vector_type(2)));
+// The running maximum of a row moves only when a score passes it by more than
+// kLazy in log2 units, so O is rescaled on few tiles; weights then reach
+// 2^(kLazy + kBias). fp16 weights carry 2^kBias so that small ones stay normal
+// binary16 numbers, with the largest below 2^15.
+template <bool kF16>
+struct PrefillWeights {
+    static constexpr float kLazy = kF16 ? 4.0f : kLazyMaxLog2;
+    static constexpr float kBias = kF16 ? 11.0f : 0.0f;
+};
 
-template <typename OutT>
+// Largest of this lane's sixteen scores. maximum (not fmax) takes the MFMA
+// results without a canonicalising instruction each; a NaN score makes its
+// row's weights NaN either way.
+__device__ inline float lane_max(const floatx16& s) {
+    float m = s[0];
+#pragma unroll
+    for (int r = 1; r < 15; r += 2) {
+        m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, s[r]), s[r + 1]);
+    }
+    return __builtin_elementwise_maximum(m, s[15]);
+}
+
+// P of one tile as the hi and lo B operands of the PV k-steps; returns this
+// lane's sum of its sixteen weights. bf16: hi = P truncated, lo = P - hi
+// rounded to nearest even. (v_dot2_f32_bf16 gives p - hi in one instruction,
+// but holds the matrix core up: beside MFMAs it costs as much as three others.)
+template <bool kF16>
+__device__ inline float prefill_weights(const floatx16& s, float scale_log2, float bias, u32x4 (&hi)[2],
+                                        u32x4 (&lo)[2]) {
+    float psum = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; r += 2) {
+        const float p0 = fast_exp2(fmaf(s[r], scale_log2, bias));
+        const float p1 = fast_exp2(fmaf(s[r + 1], scale_log2, bias));
+        psum += p0 + p1;
+        if constexpr (kF16) {
+            const f16x2_t a = {static_cast<_Float16>(p0), static_cast<_Float16>(p1)};
+            const f16x2_t b = {static_cast<_Float16>(p0 - static_cast<float>(a[0])),
+                               static_cast<_Float16>(p1 - static_cast<float>(a[1]))};
+            hi[r / 8][(r / 2) & 3] = __builtin_bit_cast(uint32_t, a);
+            lo[r / 8][(r / 2) & 3] = __builtin_bit_cast(uint32_t, b);
+        } else {
+            const uint32_t b0 = __float_as_uint(p0);
+            const uint32_t b1 = __float_as_uint(p1);
+            const bf16x2_t b = {static_cast<__bf16>(p0 - __uint_as_float(b0 & 0xffff0000u)),
+                                static_cast<__bf16>(p1 - __uint_as_float(b1 & 0xffff0000u))};
+            // High halves of p0 (low word) and p1 (high word) in one byte permute.
+            hi[r / 8][(r / 2) & 3] = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
+            lo[r / 8][(r / 2) & 3] = __builtin_bit_cast(uint32_t, b);
+        }
+    }
+    return psum;
+}
+
+template <bool kF16, int kD, typename OutT>
 __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_mfma(DecodeGeometry p, const PrefillItem* items,
-                                                                    void* out_ptr) {
-    __shared__ __attribute__((aligned(16))) PrefillTile sm[2];
+                                                                   void* out_ptr) {
+    constexpr int kQk = kD / 16;               // QK k-steps
+    constexpr int kPv = kD / 32;               // PV row blocks
+    constexpr int kHalf = kPv / 2;             // row blocks per half of PV
+    constexpr int kChunks = kD / 8;            // 16-byte chunks per row
+    constexpr int kLoadRows = 64 / kChunks;    // rows one direct load fills
+    constexpr int kLoads = 8 / kLoadRows;      // direct loads per wave of a tile's K (and of its V)
+    constexpr uint32_t kRow = 2 * kD;          // bytes
+    constexpr uint32_t kTileBytes = kTileTokens * kRow;
+    constexpr float kLazy = PrefillWeights<kF16>::kLazy;
+    constexpr float kBias = PrefillWeights<kF16>::kBias;
+    __shared__ __attribute__((aligned(256))) uint8_t sm[(kKRing + kVRing) * kTileBytes];
+    __shared__ int sm_bad[kPrefillWaves];
 
     const auto* itp = as_const(items) + blockIdx.x;
     const int b = itp->b;
     const int g = itp->g;
-    const int p0 = itp->p0;
-    const int np = itp->np;
+    const int start = itp->start;
+    const int r0 = itp->r0;
+    const int nrows = itp->nrows;
     const int row0 = itp->row0;
-    const int h0 = itp->h0;
 
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
-    const int c = lane & 15;
-    const int j = lane >> 4;
+    const int c = lane & 31;
+    const int h = lane >> 5;
     const int G = static_cast<int>(p.group);
-    const int nh = min(G - h0, kPrefillHeadsPerItem);
-    // This wave's query heads (within the group): h0 + wave and h0 + wave + 4.
-    const bool has_a = wave < nh;
-    const bool has_b = wave + kPrefillWaves < nh;
-    const int ctx_end = p0 + np;
-    const int ntiles = (ctx_end + kTileTokens - 1) / kTileTokens;
+    const int pmin = start + r0 / G;
+    const int last_tok = start + min(r0 + kPrefillRows - 1, nrows - 1) / G;
+    const int ntiles = last_tok / kTileTokens + 1;
+    // A wave past the last row only loads its share of the tiles.
+    const bool active = r0 + 32 * wave < nrows;
 
-    // Column c is position p0 + c; columns past the block repeat its last
-    // position (valid data, never written).
-    const int cc = min(c, np - 1);
-    const int col_last = p0 + cc;
-    const uint16_t* qrow = static_cast<const uint16_t*>(p.query) +
-                           (static_cast<uint64_t>(row0 + cc) * p.num_q_heads + static_cast<uint64_t>(g) * G) * 128;
-    u32x4 qa[4], qb[4];
+    // Column c is row r0 + 32 wave + c; columns past the last row repeat it
+    // (valid data, never written).
+    const int row = min(r0 + 32 * wave + c, nrows - 1);
+    const int pos = row / G;
+    const int col_last = start + pos;
+    const uint64_t qoff =
+        (static_cast<uint64_t>(row0 + pos) * p.num_q_heads + static_cast<uint64_t>(g) * G + (row - pos * G)) * kD;
+    u32x4 q[kQk];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        qa[i] = *reinterpret_cast<const u32x4*>(qrow + (h0 + min(wave, nh - 1)) * 128 + 32 * i + 8 * j);
-        qb[i] = *reinterpret_cast<const u32x4*>(qrow + (h0 + min(wave + kPrefillWaves, nh - 1)) * 128 + 32 * i + 8 * j);
+    for (int i = 0; i < kQk; ++i) {
+        q[i] = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(p.query) + qoff + 16 * i + 8 * h);
     }
-    floatx4 oa[8], ob[8];
-#pragma unroll
-    for (int n = 0; n < 8; ++n) {
-        oa[n] = floatx4{0.f, 0.f, 0.f, 0.f};
-        ob[n] = floatx4{0.f, 0.f, 0.f, 0.f};
-    }
-    float ma = -INFINITY, la = 0.f, mb = -INFINITY, lb = 0.f;
 
-    // Tile loads go from HBM straight into LDS (global_load_lds_dwordx4): one
-    // instruction fills four rows (1 KiB), lane l landing at byte 16 l of them
-    // -- row r0 + l / 16, physical chunk l % 16, which holds logical chunk
-    // (l % 16) ^ (row % 16). A tile's two 16-token halves lie in one block each
-    // (tokens_per_block is a power of two >= 16); a half past the context's
-    // last block reads that block, and rows past the context load the
-    // context's last token (finite data under weights of 0), so every address
-    // stays inside a mapped frame. With an odd group the last wave holds one
-    // head and issues all sixteen loads of a tile (K and V, rows 0 .. 31),
-    // leaving the two-head waves none to issue or wait for; otherwise wave w
-    // loads rows 8w .. 8w + 7.
+    // Tile loads go straight into LDS (global_load_lds_dwordx4): one
+    // instruction fills kLoadRows rows (1 KiB), lane l landing at byte 16 l of
+    // them -- row l / kChunks, physical chunk l % kChunks, which takes the
+    // logical chunk the row's key puts there. Wave w loads rows 8w .. 8w + 7
+    // of K and V; they lie in one block (tokens_per_block is a power of two >=
+    // 16). In a tile past the item's last token a half past that token's block
+    // reads that block and rows past the token load it again (finite data
+    // under weights of 0), so every address stays inside a mapped frame.
     const auto* trow = as_const(p.tables) + static_cast<uint64_t>(b) * p.max_nb;
-    const int last_tok = ctx_end - 1;
     const int last_blk = last_tok >> p.tpb_shift;
-    const uint8_t* kbase = p.kv_base + p.k_off;
-    const uint8_t* vbase = p.kv_base + p.v_off;
-    const bool one_loader = nh == kPrefillHeadsPerItem - 1;
-    auto load_rows = [&](int buf, int tile, int r0) {
-        const int row = r0 + (lane >> 4);
-        const int tok = min(tile * kTileTokens + row, last_tok);
-        const int half_tok0 = tile * kTileTokens + (r0 & 16);
-        const uint64_t off = static_cast<uint64_t>(trow[min(half_tok0 >> p.tpb_shift, last_blk)]) * p.block_stride +
-                             static_cast<uint64_t>(g) * p.head_stride +
-                             static_cast<uint64_t>(tok & (p.tpb - 1)) * p.token_stride +
-                             16u * static_cast<uint32_t>((lane & 15) ^ (row & 15));
-        __builtin_amdgcn_global_load_lds(kbase + off, (__attribute__((address_space(3))) void*)(&sm[buf].k[r0][0]), 16,
-                                         0, 0);
-        __builtin_amdgcn_global_load_lds(vbase + off, (__attribute__((address_space(3))) void*)(&sm[buf].v[r0][0]), 16,
-                                         0, 0);
-    };
-    auto load_tile_lds = [&](int buf, int tile) {
-        if (one_loader) {
-            if (wave == kPrefillWaves - 1) {
+    const uint8_t* kbase = p.kv_base + p.k_off + static_cast<uint64_t>(g) * p.head_stride;
+    const uint64_t kv_gap = p.v_off - p.k_off;
+    const uint32_t tstride = static_cast<uint32_t>(p.token_stride);
+    const int half_off = 16 * (wave >> 1);
+    uint32_t off_k[kLoads], off_v[kLoads];
 #pragma unroll
-                for (int q = 0; q < 8; ++q) load_rows(buf, tile, 4 * q);
-            }
+    for (int i = 0; i < kLoads; ++i) {
+        const int lr = 8 * wave + kLoadRows * i + lane / kChunks;
+        const uint32_t o = static_cast<uint32_t>(lr & 15) * tstride;
+        off_k[i] = o + 16u * static_cast<uint32_t>((lane % kChunks) ^ k_key<kD>(lr));
+        off_v[i] = o + 16u * static_cast<uint32_t>((lane % kChunks) ^ v_key<kD>(lr));
+    }
+    typedef __attribute__((address_space(3))) uint8_t lds_byte;
+    lds_byte* const lds = (lds_byte*)sm;
+    // In assembly, as the compiler would wait for every direct load before any
+    // transposed read of LDS, whichever ring slot either of them is in. The
+    // loads write no register; the s_waitcnt before each barrier covers them.
+    auto direct_load = [&](uint32_t lds_at, uint32_t off, const uint8_t* base) {
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                     :
+                     : "s"(lds_at), "v"(off), "s"(base)
+                     : "memory");
+    };
+    auto load_rows = [&](uint32_t at, int tile, const uint8_t* base, const uint32_t (&off)[kLoads]) {
+        const int tok0 = tile * kTileTokens + half_off;
+        const uint8_t* frame =
+            base + static_cast<uint64_t>(trow[min(tok0 >> p.tpb_shift, last_blk)]) * p.block_stride;
+        at += 8u * wave * kRow + static_cast<uint32_t>((uintptr_t)lds);
+        if (tok0 + 15 <= last_tok) {
+            frame += static_cast<uint64_t>(tok0 & (p.tpb - 1)) * p.token_stride;
+#pragma unroll
+            for (int i = 0; i < kLoads; ++i) direct_load(at + 1024u * i, off[i], frame);
         } else {
 #pragma unroll
-            for (int q = 0; q < 2; ++q) load_rows(buf, tile, 8 * wave + 4 * q);
+            for (int i = 0; i < kLoads; ++i) {
+                const int lr = (8 * wave + kLoadRows * i + lane / kChunks) & 15;
+                const uint32_t in = static_cast<uint32_t>(min(tok0 + lr, last_tok)) & (p.tpb - 1);
+                direct_load(at + 1024u * i, off[i] + (in - static_cast<uint32_t>(lr)) * tstride, frame);
+            }
         }
     };
-
-    auto read_k = [&](int buf, u32x4 (&kf)[2][4]) {
+    auto load_k = [&](int slot, int tile) { load_rows(slot * kTileBytes, tile, kbase, off_k); };
+    auto load_v = [&](int slot, int tile) { load_rows((kKRing + slot) * kTileBytes, tile, kbase + kv_gap, off_v); };
+    // Fragment addresses: the chunks one lane reads of a tile differ by XOR of
+    // constant bits (and rows 8 and 16 further), so one address serves them all.
+    const uint32_t k_lane = static_cast<uint32_t>(c * kRow + 16 * (h ^ k_key<kD>(c)));
+    const int vi = lane & 15;
+    const int vrow = 4 * h + (vi >> 2);
+    const uint32_t v_lane = static_cast<uint32_t>(
+        kKRing * kTileBytes + vrow * kRow + 16 * ((2 * ((lane >> 4) & 1) + ((vi & 3) >> 1)) ^ v_key<kD>(vrow)) +
+        8 * (vi & 1));
+    static_assert(kKRing * kTileBytes % 256 == 0 && kTileBytes % 256 == 0, "XOR of chunk bits must not carry");
+    // K operands of k-steps x kQk / 2 .. (x + 1) kQk / 2 - 1.
+    auto read_k = [&](int slot, int x, u32x4 (&kf)[kQk / 2]) {
+        const uint32_t a = k_lane + static_cast<uint32_t>(slot) * kTileBytes;
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int row = 16 * u + (c >> 2) + 4 * (c & 3);
-                kf[u][i] = lds16(&sm[buf].k[row][swz(row, 16 * j + 64 * i)]);
-            }
-    };
-    auto read_v = [&](int buf, u32x4 (&vf)[8]) {
-#pragma unroll
-        for (int n = 0; n < 8; ++n) {
-            u32x4 a;
-#pragma unroll
-            for (int hh = 0; hh < 2; ++hh) {
-                const int row = 4 * ((c >> 2) + 4 * hh) + j;
-                const v4i16 t = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                    (v4i16 __attribute__((address_space(3)))*)(&sm[buf].v[row][swz(row, 2 * (16 * n + 4 * (c & 3)))]));
-                a[2 * hh] = __builtin_bit_cast(uint2v, t)[0];
-                a[2 * hh + 1] = __builtin_bit_cast(uint2v, t)[1];
-            }
-            vf[n] = a;
+        for (int i = 0; i < kQk / 2; ++i) {
+            kf[i] = *(const __attribute__((address_space(3))) u32x4*)(lds + (a ^ (32u * (i + x * kQk / 2))));
         }
     };
-    // Causal mask of tile t for both heads: column c sees tokens <= col_last.
-    auto mask2 = [&](floatx4 (&sa)[2], floatx4 (&sb)[2], int t) {
+    // V operands of row blocks x kHalf .. (x + 1) kHalf - 1, both k-steps.
+    auto read_v = [&](int slot, int x, u32x4 (&vf)[kHalf][2]) {
+        const uint32_t a = v_lane + static_cast<uint32_t>(slot) * kTileBytes;
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int n = 0; n < kHalf; ++n)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const bool out = t * kTileTokens + j + 16 * u + 4 * r > col_last;
-                sa[u][r] = out ? -INFINITY : sa[u][r];
-                sb[u][r] = out ? -INFINITY : sb[u][r];
-            }
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    // Eight rows further the key changes by 2 (both head dims).
+                    const v4i16 t = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4i16 __attribute__((address_space(3)))*)(
+                        lds + ((a ^ (64u * (n + x * kHalf)) ^ (32u * e)) + (16 * ks + 8 * e) * kRow)));
+                    vf[n][ks][2 * e] = __builtin_bit_cast(uint2v, t)[0];
+                    vf[n][ks][2 * e + 1] = __builtin_bit_cast(uint2v, t)[1];
+                }
     };
 
-    // Software pipeline over tiles. Iteration t issues PV(t) (P and V of tile
-    // t already in registers) in one basic block with QK and the softmax of
-    // tile t + 1, which do not depend on it, so the MFMAs of one overlap the
-    // VALU work of the other; tile t + 2 is loaded into the LDS buffer tile t
-    // used, and every wave waits for its loads before the iteration's closing
-    // barrier. Tiles from t_diag on reach the block's first
-    // position and take the causal mask; the loop is split there so the
-    // others carry no mask code. A wave with two query heads runs both in one
-    // block; a wave with one (the last wave of an odd group) runs a
-    // one-head copy of the loop, leaving its SIMD's issue slots to the
-    // other workgroup's wave there.
-    const int t_diag = (p0 + 1) / kTileTokens;
-    const int last_tile = ntiles - 1;
-    auto run = [&](auto two_heads) {
-        constexpr bool kTwo = decltype(two_heads)::value;
-        u32x4 kf[2][4], vf[8];
-        floatx4 sa[2], sb[2];
-        u32x4 ahi, alo, bhi, blo;
-        float alpha_a, alpha_b = 1.0f;
-        // A direct load has landed in LDS once vmcnt counts it done: each wave
-        // waits for all of its loads (s_waitcnt 0) before the barrier that
-        // hands the tile to the other waves.
-        load_tile_lds(0, 0);
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        if (last_tile >= 1) load_tile_lds(1, 1);
-        read_k(0, kf);
-        read_v(0, vf);
-        qk_tile(kf, qa, sa);
-        if constexpr (kTwo) qk_tile(kf, qb, sb);
-        if (t_diag == 0) mask2(sa, sb, 0);
-        softmax_p<false, false, true>(sa, p.scale_log2, ma, la, ahi, alo, alpha_a);
-        if constexpr (kTwo) softmax_p<false, false, true>(sb, p.scale_log2, mb, lb, bhi, blo, alpha_b);
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        // O is rescaled for tile t's maximum just before PV(t) accumulates
-        // into it, skipped when no column's maximum moved (the factor is then
-        // exactly 1); the branch sits at the top of the iteration, outside
-        // the block above. The maximum moves lazily (softmax_p's kLazy: only
-        // past kLazyMaxLog2 above the current one), so after the first tiles
-        // almost no iteration rescales.
-        auto rescale = [&]() {
-            if (__builtin_amdgcn_ballot_w64(alpha_a != 1.0f || alpha_b != 1.0f) != 0) {
+    const int t_diag = (pmin + 1) / kTileTokens;  // first tile that needs masks
+    const float lazy_raw = kLazy / p.scale_log2;
+    floatx16 o[kPv];
+    float lsum;
+
+    // One pass over the item's tiles. `careful` (a second pass, taken when the
+    // first left a non-finite output) multiplies the masked tiles' V column by
+    // column with the values past the column's position cleared: V rows a row
+    // does not see meet weights of 0, but 0 x inf would still poison it.
+    auto run = [&](bool careful) {
+        struct Weights { u32x4 hi[2], lo[2]; };
+        // Running maximum m of the column as bias = kBias - m and thr, the raw
+        // score past which it moves; thr is -inf until a score was seen.
+        float thr = -INFINITY, bias = kBias, alpha = 1.0f, lm = -INFINITY;
+        bool rescale_o = false;
+        lsum = 0.f;
 #pragma unroll
-                for (int n = 0; n < 8; ++n) {
-                    oa[n] *= alpha_a;
-                    if constexpr (kTwo) ob[n] *= alpha_b;
+        for (int n = 0; n < kPv; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[n][r] = 0.f;
+        auto qk = [&](const u32x4 (&kf)[kQk / 2], int x, floatx16& sc) {
+            if (x == 0) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sc[r] = 0.f;
+            }
+#pragma unroll
+            for (int i = 0; i < kQk / 2; ++i) sc = mfma32<kF16>(kf[i], q[i + x * kQk / 2], sc);
+        };
+        auto pv = [&](const u32x4 (&vf)[kHalf][2], int x, const Weights& w) {
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+                for (int n = 0; n < kHalf; ++n) o[n + x * kHalf] = mfma32<kF16>(vf[n][ks], w.hi[ks], o[n + x * kHalf]);
+#pragma unroll
+                for (int n = 0; n < kHalf; ++n) o[n + x * kHalf] = mfma32<kF16>(vf[n][ks], w.lo[ks], o[n + x * kHalf]);
+            }
+        };
+        auto pv_careful = [&](const u32x4 (&vf)[kHalf][2], int x, const Weights& w, int t) {
+            for (int col = 0; col < 32; ++col) {
+                const bool mine = c == col;
+                const int lim = __builtin_amdgcn_readlane(col_last, col) - t * kTileTokens - 4 * h;
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) {
+                    u32x4 hi, lo, keep;
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        const int tok = 16 * ks + 8 * (d >> 1) + 2 * (d & 1);  // of elements 2d, 2d + 1
+                        hi[d] = mine ? w.hi[ks][d] : 0u;
+                        lo[d] = mine ? w.lo[ks][d] : 0u;
+                        keep[d] = (tok <= lim ? 0x0000ffffu : 0u) | (tok + 1 <= lim ? 0xffff0000u : 0u);
+                    }
+#pragma unroll
+                    for (int m = 0; m < kHalf; ++m) {
+                        const int n = m + x * kHalf;
+                        const floatx16 a = mfma32<kF16>(vf[m][ks] & keep, lo, mfma32<kF16>(vf[m][ks] & keep, hi, o[n]));
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) o[n][r] = mine ? a[r] : o[n][r];
+                    }
                 }
             }
         };
-        auto step = [&](int t, auto masked) {
-            const int nb = (t + 1) & 1;
-            rescale();
-            // Tile t + 2; near the end the last tile again, which lands in a
-            // buffer no later iteration reads.
-            // Tile t + 2 into the buffer tile t used (read at iteration t - 1).
-            if (t + 2 <= last_tile) load_tile_lds(t & 1, t + 2);
-            read_k(nb, kf);
-            qk_tile(kf, qa, sa);
-            if constexpr (kTwo) qk_tile(kf, qb, sb);
-            pv_tile(vf, ahi, alo, oa);
-            if constexpr (kTwo) pv_tile(vf, bhi, blo, ob);
-            read_v(nb, vf);
-            if constexpr (decltype(masked)::value) mask2(sa, sb, t + 1);
-            softmax_p<false, false, true>(sa, p.scale_log2, ma, la, ahi, alo, alpha_a);
-            if constexpr (kTwo) softmax_p<false, false, true>(sb, p.scale_log2, mb, lb, bhi, blo, alpha_b);
-            // Schedule: the QK MFMAs first, then the PV MFMAs spread over the
-            // softmax's VALU work.
-            constexpr int kHeads = kTwo ? 2 : 1;
+        auto mask = [&](floatx16& sc, int t) {
 #pragma unroll
-            for (int k = 0; k < 8 * kHeads; ++k) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-#pragma unroll
-            for (int k = 0; k < 16 * kHeads; ++k) {
-                __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            for (int r = 0; r < 16; ++r) {
+                sc[r] = t * kTileTokens + (r & 3) + 8 * (r >> 2) + 4 * h > col_last ? -INFINITY : sc[r];
             }
+        };
+        auto rescale = [&]() {
+            if (rescale_o) {
+#pragma unroll
+                for (int n = 0; n < kPv; ++n) o[n] *= alpha;
+            }
+        };
+        // Moves the maxima that a score of the tile passes by more than kLazy
+        // (lm: this lane's largest). O still lacks the previous tile's product
+        // then, so it is scaled at the next call.
+        auto raise = [&]() {
+            const uint64_t up = __builtin_amdgcn_ballot_w64(lm > thr);
+            if (!rescale_o && up == 0) return;
+            rescale();
+            rescale_o = up != 0;
+            const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(lm), __float_as_uint(lm), false, false);
+            const float mt = fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
+            const bool move = mt > thr;
+            const float to = kBias - mt * p.scale_log2;
+            alpha = move && thr != -INFINITY ? fast_exp2(to - bias) : 1.0f;
+            bias = move ? to : bias;
+            thr = move ? mt + lazy_raw : thr;
+            lsum *= alpha;
+        };
+
+        floatx16 sa, sb;
+        Weights wa, wb;
+        u32x4 va[kHalf][2];  // first half of the V operands the next PV takes
+        // A direct load has landed in LDS once vmcnt counts it done: each wave
+        // waits for all of its loads before the barrier that hands the tiles
+        // to the other waves.
+        load_k(0, 0);
+        load_v(0, 0);
+        if (ntiles > 1) load_k(1, 1);
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (active) {
+            u32x4 k0[kQk / 2], k1[kQk / 2];
+            read_k(0, 0, k0);
+            read_k(0, 1, k1);
+            qk(k0, 0, sa);
+            qk(k1, 1, sa);
+            if (t_diag == 0) mask(sa, 0);
+            lm = lane_max(sa);
+        }
+        __syncthreads();
+        int vslot = 0;  // ring slot of V(t)
+        // Step t: the softmax of tile t (s -> w), with QK of tile t + 1 (-> s2)
+        // and PV of tile t - 1 (w0) around it: none of the three depends on
+        // another, so the matrix products run beside the vector work.
+        auto step = [&](int t, const floatx16& s, Weights& w, floatx16& s2, const Weights& w0, auto first, auto masked) {
+            constexpr bool kFirst = decltype(first)::value;
+            constexpr bool kMasked = decltype(masked)::value;
+            const int vprev = vslot == 0 ? kVRing - 1 : vslot - 1;
+            const int vnext = vslot == kVRing - 1 ? 0 : vslot + 1;
+            load_v(vnext, t + 1);
+            if (t + 2 < ntiles) load_k(t & 1, t + 2);
+            if (active) {
+                raise();
+                u32x4 k0[kQk / 2], k1[kQk / 2], vb[kHalf][2];
+                read_k((t + 1) & 1, 0, k0);
+                if constexpr (!kFirst) {
+                    if (kMasked && careful) {
+                        pv_careful(va, 0, w0, t - 1);
+                    } else {
+                        pv(va, 0, w0);
+                    }
+                }
+                read_k((t + 1) & 1, 1, k1);
+                qk(k0, 0, s2);
+                if constexpr (!kFirst) read_v(vprev, 1, vb);
+                qk(k1, 1, s2);
+                lsum += prefill_weights<kF16>(s, p.scale_log2, bias, w.hi, w.lo);
+                if constexpr (!kFirst) {
+                    if (kMasked && careful) {
+                        pv_careful(vb, 1, w0, t - 1);
+                    } else {
+                        pv(vb, 1, w0);
+                    }
+                }
+                read_v(vslot, 0, va);
+                if constexpr (kMasked) mask(s2, t + 1);
+                lm = lane_max(s2);
+            }
+            vslot = vnext;
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
         };
         int t = 0;
-        for (; t + 1 < min(t_diag, ntiles); ++t) step(t, std::false_type{});
-        for (; t + 1 < ntiles; ++t) step(t, std::true_type{});
-        rescale();
-        pv_tile(vf, ahi, alo, oa);
-        if constexpr (kTwo) pv_tile(vf, bhi, blo, ob);
+        if (ntiles > 1) {
+            step(0, sa, wa, sb, wa, std::true_type{}, std::true_type{});
+            sa = sb;
+            for (t = 1; t + 2 < min(t_diag, ntiles); t += 2) {
+                step(t, sa, wb, sb, wa, std::false_type{}, std::false_type{});
+                step(t + 1, sb, wa, sa, wb, std::false_type{}, std::false_type{});
+            }
+            for (; t < ntiles - 1; ++t) {
+                step(t, sa, wb, sb, wa, std::false_type{}, std::true_type{});
+                sa = sb;
+                wa = wb;
+            }
+        }
+        // Tile t = ntiles - 1: PV of the tile before, its softmax and its own PV.
+        if (active) {
+            raise();
+            u32x4 vb[kHalf][2];
+            if (t > 0) {
+                read_v(vslot == 0 ? kVRing - 1 : vslot - 1, 1, vb);
+                if (careful) {
+                    pv_careful(va, 0, wa, t - 1);
+                    pv_careful(vb, 1, wa, t - 1);
+                } else {
+                    pv(va, 0, wa);
+                    pv(vb, 1, wa);
+                }
+            }
+            rescale();
+            lsum += prefill_weights<kF16>(sa, p.scale_log2, bias, wa.hi, wa.lo);
+            read_v(vslot, 0, va);
+            read_v(vslot, 1, vb);
+            if (careful) {
+                pv_careful(va, 0, wa, t);
+                pv_careful(vb, 1, wa, t);
+            } else {
+                pv(va, 0, wa);
+                pv(vb, 1, wa);
+            }
+            const auto both =
+                __builtin_amdgcn_permlane32_swap(__float_as_uint(lsum), __float_as_uint(lsum), false, false);
+            lsum = __uint_as_float(both[0]) + __uint_as_float(both[1]);
+        }
     };
-    if (has_b) {
-        run(std::true_type{});
-    } else {
-        run(std::false_type{});
+    run(false);
+    float nonfinite = 0.f;
+    if (active) {
+#pragma unroll
+        for (int n = 0; n < kPv; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) nonfinite = fmaf(o[n][r], 0.f, nonfinite);
     }
+    const bool wave_bad = __builtin_amdgcn_ballot_w64(nonfinite != 0.f) != 0;
+    if (lane == 0) sm_bad[wave] = wave_bad ? 1 : 0;
+    __syncthreads();
+    int bad = 0;
+#pragma unroll
+    for (int w = 0; w < kPrefillWaves; ++w) bad |= sm_bad[w];
+    if (__builtin_amdgcn_readfirstlane(bad) != 0) run(true);
 
-    OutT* out = static_cast<OutT*>(out_ptr);
-    // C register r of PV MFMA n in lane (c, j) is O[column c][dim 16n + 4j +
-    // r]: four contiguous outputs per n, stored as one vector, so a store
-    // instruction writes 16 contiguous dims (4 lanes) of each of its 16 rows
-    // (one 2-byte store per element took a fifth of the kernel).
-    auto write = [&](int hq, const floatx4 (&o)[8], float l) {
-        if (c >= np) return;
-        OutT* dst = out + (static_cast<uint64_t>(row0 + c) * p.num_q_heads + static_cast<uint64_t>(g) * G + hq) * 128 +
-                    4 * j;
+    if (r0 + 32 * wave + c >= nrows) return;
+    // C register r of PV block n in lane (c, h) is O[column c][dim 32n +
+    // (r % 4) + 8 (r / 4) + 4h]: four contiguous outputs per r / 4, stored as
+    // one vector (one 2-byte store per element took a fifth of the kernel).
+    OutT* dst = static_cast<OutT*>(out_ptr) + qoff + 4 * h;
+    const float inv = 1.0f / lsum;
 #pragma unroll
-        for (int n = 0; n < 8; ++n) {
+    for (int n = 0; n < kPv; ++n) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            floatx4 x;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[r] = o[n][4 * k + r] * inv;
+            OutT* at = dst + 32 * n + 8 * k;
             if constexpr (sizeof(OutT) == 4) {
-                u32x4 a;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) a[r] = __float_as_uint(o[n][r] / l);
-                *reinterpret_cast<u32x4*>(dst + 16 * n) = a;
+                *reinterpret_cast<floatx4*>(at) = x;
             } else {
                 uint2v a;
 #pragma unroll
-                for (int k = 0; k < 2; ++k) {
-                    const OutT lo_v = from_float<OutT>(o[n][2 * k] / l);
-                    const OutT hi_v = from_float<OutT>(o[n][2 * k + 1] / l);
-                    a[k] = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, lo_v)) |
-                           (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, hi_v)) << 16);
+                for (int r = 0; r < 2; ++r) {
+                    if constexpr (std::is_same_v<OutT, uint16_t>) {
+                        const bf16x2_t y = {static_cast<__bf16>(x[2 * r]), static_cast<__bf16>(x[2 * r + 1])};
+                        a[r] = __builtin_bit_cast(uint32_t, y);
+                    } else {
+                        const f16x2_t y = {static_cast<_Float16>(x[2 * r]), static_cast<_Float16>(x[2 * r + 1])};
+                        a[r] = __builtin_bit_cast(uint32_t, y);
+                    }
                 }
-                *reinterpret_cast<uint2v*>(dst + 16 * n) = a;
+                *reinterpret_cast<uint2v*>(at) = a;
             }
         }
-    };
-    la = sum_over_j(la);
-    lb = sum_over_j(lb);
-    if (has_a) write(h0 + wave, oa, la);
-    if (has_b) write(h0 + wave + kPrefillWaves, ob, lb);
+    }
 }
 
 bool prefill_mfma_supported(const DecodeGeometry& g, uint32_t kv_dtype, uintptr_t query_addr, uintptr_t kv_base_addr,
@@ -334,8 +544,26 @@ bool prefill_mfma_supported(const DecodeGeometry& g, uint32_t kv_dtype, uintptr_
     const bool aligned = (g.block_stride % 16 == 0) && (g.k_off % 16 == 0) && (g.v_off % 16 == 0) &&
                          (g.token_stride % 16 == 0) && (g.head_stride % 16 == 0) && (kv_base_addr % 16 == 0) &&
                          (query_addr % 16 == 0) && (out_addr % 16 == 0);
-    return kv_dtype == QVP_DTYPE_BF16 && g.head_dim == 128 && g.group >= 1 && g.group <= 16 && pow2 && g.tpb >= 16 &&
-           aligned;
+    // A lane's offset inside a 16-token half is kept in 32 bits.
+    return (kv_dtype == QVP_DTYPE_BF16 || kv_dtype == QVP_DTYPE_F16) && (g.head_dim == 128 || g.head_dim == 64) &&
+           pow2 && g.tpb >= 16 && aligned && g.token_stride * g.tpb <= 0x7fffffffu;
+}
+
+template <bool kF16, int kD>
+void launch_prefill(const DecodeGeometry& g, const PrefillItem* items, uint32_t count, uint32_t out_dtype, void* out,
+                    hipStream_t s) {
+    const dim3 grid(count), block(kPrefillThreads);
+    switch (out_dtype) {
+        case QVP_DTYPE_F32:
+            hipLaunchKernelGGL((prefill_mfma<kF16, kD, float>), grid, block, 0, s, g, items, out);
+            break;
+        case QVP_DTYPE_BF16:
+            hipLaunchKernelGGL((prefill_mfma<kF16, kD, uint16_t>), grid, block, 0, s, g, items, out);
+            break;
+        default:
+            hipLaunchKernelGGL((prefill_mfma<kF16, kD, _Float16>), grid, block, 0, s, g, items, out);
+            break;
+    }
 }
 
 uint32_t log2_u32(uint32_t x) {
@@ -485,28 +713,28 @@ extern "C" int qvp_paged_prefill(const qvp_prefill_args* a, void* stream) {
     }
 
     // Work items, longest context first.
-    const uint32_t G = g.group;
-    const uint32_t head_sets = (G + qvp::kPrefillHeadsPerItem - 1) / qvp::kPrefillHeadsPerItem;
+    const uint64_t G = g.group;
     std::vector<qvp::PrefillItem> items;
     uint32_t row = 0;
     for (uint32_t sq = 0; sq < v.num_seqs; ++sq) {
         const uint32_t start = a->q_start[sq];
-        const uint32_t end = static_cast<uint32_t>(lens[sq]);
-        for (uint32_t p0 = start; p0 < end; p0 += qvp::kPrefillPositions) {
-            const uint32_t np = std::min<uint32_t>(qvp::kPrefillPositions, end - p0);
+        const uint32_t fresh = static_cast<uint32_t>(lens[sq]) - start;
+        if (fresh * G > 0x7fffffffu - qvp::kPrefillRows) return fail(QVP_ERR_INVALID_ARGUMENT, "too many new tokens");
+        const uint32_t nrows = static_cast<uint32_t>(fresh * G);
+        for (uint32_t r0 = 0; r0 < nrows; r0 += qvp::kPrefillRows) {
             for (uint32_t kv = 0; kv < a->num_kv_heads; ++kv) {
-                for (uint32_t hs = 0; hs < head_sets; ++hs) {
-                    items.push_back(qvp::PrefillItem{static_cast<int32_t>(sq), static_cast<int32_t>(kv),
-                                                     static_cast<int32_t>(p0), static_cast<int32_t>(np),
-                                                     static_cast<int32_t>(row + (p0 - start)),
-                                                     static_cast<int32_t>(hs * qvp::kPrefillHeadsPerItem)});
-                }
+                items.push_back(qvp::PrefillItem{static_cast<int32_t>(sq), static_cast<int32_t>(kv),
+                                                 static_cast<int32_t>(start), static_cast<int32_t>(r0),
+                                                 static_cast<int32_t>(nrows), static_cast<int32_t>(row)});
             }
         }
-        row += end - start;
+        row += fresh;
     }
-    std::stable_sort(items.begin(), items.end(), [](const qvp::PrefillItem& x, const qvp::PrefillItem& y) {
-        return x.p0 + x.np > y.p0 + y.np;
+    const auto last_token = [G](const qvp::PrefillItem& x) {
+        return x.start + (std::min(x.r0 + qvp::kPrefillRows, x.nrows) - 1) / static_cast<int32_t>(G);
+    };
+    std::stable_sort(items.begin(), items.end(), [&](const qvp::PrefillItem& x, const qvp::PrefillItem& y) {
+        return last_token(x) > last_token(y);
     });
     if (items.size() > 0x7fffffffu) return fail(QVP_ERR_INVALID_ARGUMENT, "too many prefill items");
     const size_t ints = items.size() * (sizeof(qvp::PrefillItem) / sizeof(int32_t));
@@ -542,19 +770,14 @@ extern "C" int qvp_paged_prefill(const qvp_prefill_args* a, void* stream) {
     plan.staging_pending = true;
 
     const auto* dev_items = reinterpret_cast<const qvp::PrefillItem*>(plan.device);
-    const dim3 grid(static_cast<unsigned>(items.size()));
-    switch (a->out_dtype) {
-        case QVP_DTYPE_F32:
-            hipLaunchKernelGGL(qvp::prefill_mfma<float>, grid, dim3(qvp::kPrefillThreads), 0, s, g, dev_items, a->out);
-            break;
-        case QVP_DTYPE_BF16:
-            hipLaunchKernelGGL(qvp::prefill_mfma<uint16_t>, grid, dim3(qvp::kPrefillThreads), 0, s, g, dev_items,
-                               a->out);
-            break;
-        default:
-            hipLaunchKernelGGL(qvp::prefill_mfma<_Float16>, grid, dim3(qvp::kPrefillThreads), 0, s, g, dev_items,
-                               a->out);
-            break;
+    const uint32_t count = static_cast<uint32_t>(items.size());
+    const bool f16 = a->kv_dtype == QVP_DTYPE_F16;
+    if (g.head_dim == 128) {
+        f16 ? qvp::launch_prefill<true, 128>(g, dev_items, count, a->out_dtype, a->out, s)
+            : qvp::launch_prefill<false, 128>(g, dev_items, count, a->out_dtype, a->out, s);
+    } else {
+        f16 ? qvp::launch_prefill<true, 64>(g, dev_items, count, a->out_dtype, a->out, s)
+            : qvp::launch_prefill<false, 64>(g, dev_items, count, a->out_dtype, a->out, s);
     }
     QVP_HIP(hipGetLastError());
     // The kernel reads the packed block tables: a later pack into this slot
