@@ -127,8 +127,7 @@ int qvp_event_elapsed_ms(float* ms, void* start, void* stop);
  * schedule is then cached on the device) with a caller workspace,
  * qvp_append_kv, qvp_copy_blocks, qvp_swap_gather / qvp_swap_scatter,
  * qvp_fill_bytes and device-to-device copies. qvp_pack, qvp_paged_prefill and
- * qvp_mrope_positions upload host-built lists on every call and are not
- * captured. The kernels reset their own merge counters, so a graph may be
+ * qvp_mrope_positions upload host-built lists and are not captured. The kernels reset their own merge counters, so a graph may be
  * replayed any number of times; it reads and writes the buffers it was
  * captured with, so a captured decode stays valid until the second qvp_pack
  * after the capture on its batch reuses the packed buffer it reads. */

@@ -113,16 +113,30 @@ struct qvp_schedule {
     qvp_reader reader;  // last decode that read `device`
 };
 
-// Work list of a causal prefill over one packed batch (rebuilt per call: the
-// first new position of each sequence is a call argument), and the private
-// per-position batch of the prefill's decode-kernel path.
+// Work list of a causal prefill over one packed batch, kept while the pack,
+// the first new positions and the grouping stay the same (a model's layers),
+// the workspace of its split items, and the private per-position batch of the
+// prefill's decode-kernel path.
 struct qvp_prefill_plan {
-    int32_t* staging{nullptr};
-    size_t staging_cap{0};  // int32 elements
+    void* staging{nullptr};
+    size_t staging_cap{0};  // bytes, as the other capacities here
     hipEvent_t staging_done{nullptr};
     bool staging_pending{false};
-    int32_t* device{nullptr};
+    void* device{nullptr};
     size_t device_cap{0};
+    // counters[num_parts], then the (m, l) and O of every part.
+    void* parts{nullptr};
+    size_t parts_cap{0};
+    bool parts_clean{false};  // the counters are zero between launches
+    uint32_t num_parts{0};
+    bool valid{false};
+    uint32_t num_items{0};
+    hipStream_t stream{nullptr};  // the list was uploaded on
+    uint64_t generation{0};
+    uint32_t group{0};
+    uint32_t num_kv_heads{0};
+    std::vector<uint32_t> q_start;
+    qvp_reader reader;  // last prefill that read the list and used the parts
     qvp_batch* virt{nullptr};
 };
 

@@ -28,6 +28,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <cmath>
 #include <type_traits>
 #include <cstring>
 #include <vector>
@@ -64,14 +65,13 @@ __device__ inline floatx16 mfma32(const u32x4& a, const u32x4& b, floatx16 c) {
     }
 }
 
-// K and V tiles in LDS: rows as in the frame (token-major), K in a ring of two
-// tiles, V in a ring of three. ds_read_b64_tr_b16 hands lane i of each 16-lane
+// K and V tiles in LDS: rows as in the frame (token-major), each in a ring of
+// four tiles (tile t in slot t % 4). ds_read_b64_tr_b16 hands lane i of each 16-lane
 // group element i % 4 of the 8 bytes that lane 4e + i / 4 of the group
 // addressed, as element e: with the group's lanes on tokens t .. t + 3 (by
 // i / 4) and 16 dims, lane i gets dim i of the four tokens, half of a PV
 // operand.
-constexpr int kKRing = 2;
-constexpr int kVRing = 3;
+constexpr int kRing = 4;
 // The LDS rows hold their 16-byte chunks XOR-permuted by row, so that the 64
 // lanes of a read spread over the banks: chunk x of row r lies at x ^ key(r).
 // K is read a chunk of 32 rows at a time, V four neighbouring chunks of eight
@@ -93,8 +93,23 @@ struct PrefillItem {
     int32_t r0;     // first row of the item
     int32_t nrows;  // rows of (b, g): new positions x G
     int32_t row0;   // query / output row of the first new position
+    int32_t t0, t1;  // tiles of the rows' context
+    // An item that holds all of its rows' tiles (nparts 1) writes their output.
+    // Otherwise it is one of nparts pieces: its result goes to workspace slot
+    // `slot`, the pieces' slots are slot0 .. slot0 + nparts - 1, and the
+    // workgroup that completes counters[slot0] merges them.
+    int32_t slot, slot0, nparts;
+    int32_t pad;
 };
-static_assert(sizeof(PrefillItem) == 6 * sizeof(int32_t), "PrefillItem is six int32");
+static_assert(sizeof(PrefillItem) == 12 * sizeof(int32_t), "PrefillItem is twelve int32");
+
+// Results of split items: per slot and wave, (m, l) of its 32 rows and their O
+// as the lanes hold it, two dims per lane and store (512 contiguous bytes).
+struct PrefillParts {
+    int32_t* counters;
+    uint64_t* ml;   // [slot][wave][32]
+    uint64_t* acc;  // [slot][wave][kPv x 8][64 lanes]
+};
 
 template <typename T>
 __device__ inline const __attribute__((address_space(4))) T* as_const(const T* ptr) {
@@ -157,7 +172,7 @@ __device__ inline float prefill_weights(const floatx16& s, float scale_log2, flo
 
 template <bool kF16, int kD, typename OutT>
 __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_mfma(DecodeGeometry p, const PrefillItem* items,
-                                                                   void* out_ptr) {
+                                                                   PrefillParts parts, void* out_ptr) {
     constexpr int kQk = kD / 16;               // QK k-steps
     constexpr int kPv = kD / 32;               // PV row blocks
     constexpr int kHalf = kPv / 2;             // row blocks per half of PV
@@ -168,7 +183,7 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_mfma(DecodeGeometr
     constexpr uint32_t kTileBytes = kTileTokens * kRow;
     constexpr float kLazy = PrefillWeights<kF16>::kLazy;
     constexpr float kBias = PrefillWeights<kF16>::kBias;
-    __shared__ __attribute__((aligned(256))) uint8_t sm[(kKRing + kVRing) * kTileBytes];
+    __shared__ __attribute__((aligned(256))) uint8_t sm[2 * kRing * kTileBytes];
     __shared__ int sm_bad[kPrefillWaves];
 
     const auto* itp = as_const(items) + blockIdx.x;
@@ -178,6 +193,9 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_mfma(DecodeGeometr
     const int r0 = itp->r0;
     const int nrows = itp->nrows;
     const int row0 = itp->row0;
+    const int t0 = itp->t0;
+    const int t1 = itp->t1;
+    const int nparts = itp->nparts;
 
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
@@ -186,7 +204,6 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_mfma(DecodeGeometr
     const int G = static_cast<int>(p.group);
     const int pmin = start + r0 / G;
     const int last_tok = start + min(r0 + kPrefillRows - 1, nrows - 1) / G;
-    const int ntiles = last_tok / kTileTokens + 1;
     // A wave past the last row only loads its share of the tiles.
     const bool active = r0 + 32 * wave < nrows;
 
@@ -207,75 +224,85 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_mfma(DecodeGeometr
     // instruction fills kLoadRows rows (1 KiB), lane l landing at byte 16 l of
     // them -- row l / kChunks, physical chunk l % kChunks, which takes the
     // logical chunk the row's key puts there. Wave w loads rows 8w .. 8w + 7
-    // of K and V; they lie in one block (tokens_per_block is a power of two >=
-    // 16). In a tile past the item's last token a half past that token's block
-    // reads that block and rows past the token load it again (finite data
-    // under weights of 0), so every address stays inside a mapped frame.
+    // of K and V; they lie in one 16-token half, and that in one block
+    // (tokens_per_block is a power of two >= 16). Past the half of the item's
+    // last token that half is loaded again, and its rows past the token load
+    // the token's (finite data under weights of 0), so every address stays
+    // inside a mapped frame.
     const auto* trow = as_const(p.tables) + static_cast<uint64_t>(b) * p.max_nb;
-    const int last_blk = last_tok >> p.tpb_shift;
     const uint8_t* kbase = p.kv_base + p.k_off + static_cast<uint64_t>(g) * p.head_stride;
     const uint64_t kv_gap = p.v_off - p.k_off;
     const uint32_t tstride = static_cast<uint32_t>(p.token_stride);
+    const uint32_t bstride = static_cast<uint32_t>(p.block_stride);
     const int half_off = 16 * (wave >> 1);
+    const int last_half = last_tok & ~15;
+    auto half_of = [&](int tile) { return min(tile * kTileTokens + half_off, last_half); };
+    auto block_of = [&](int tile) { return trow[half_of(tile) >> p.tpb_shift]; };
+    auto frame_of = [&](int tile, int blk) {
+        return kbase + static_cast<uint64_t>(static_cast<uint32_t>(blk)) * bstride +
+               static_cast<uint32_t>(half_of(tile) & (p.tpb - 1)) * tstride;
+    };
+    // The lane's offsets from that row; `end` for the last half.
     uint32_t off_k[kLoads], off_v[kLoads];
+    auto offsets = [&](uint32_t (&off)[kLoads], bool v, int end) {
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-        const int lr = 8 * wave + kLoadRows * i + lane / kChunks;
-        const uint32_t o = static_cast<uint32_t>(lr & 15) * tstride;
-        off_k[i] = o + 16u * static_cast<uint32_t>((lane % kChunks) ^ k_key<kD>(lr));
-        off_v[i] = o + 16u * static_cast<uint32_t>((lane % kChunks) ^ v_key<kD>(lr));
-    }
+        for (int i = 0; i < kLoads; ++i) {
+            const int lr = 8 * wave + kLoadRows * i + lane / kChunks;
+            const int key = v ? v_key<kD>(lr) : k_key<kD>(lr);
+            off[i] = static_cast<uint32_t>(min(lr & 15, end)) * tstride + 16u * static_cast<uint32_t>((lane % kChunks) ^ key);
+        }
+    };
     typedef __attribute__((address_space(3))) uint8_t lds_byte;
     lds_byte* const lds = (lds_byte*)sm;
+    const uint32_t lds_rows = static_cast<uint32_t>((uintptr_t)lds) + 8u * wave * kRow;
     // In assembly, as the compiler would wait for every direct load before any
     // transposed read of LDS, whichever ring slot either of them is in. The
     // loads write no register; the s_waitcnt before each barrier covers them.
-    auto direct_load = [&](uint32_t lds_at, uint32_t off, const uint8_t* base) {
+    auto load_rows = [&](uint32_t at, const uint8_t* frame, const uint32_t (&off)[kLoads]) {
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                      :
-                     : "s"(lds_at), "v"(off), "s"(base)
+                     : "s"(at), "v"(off[0]), "s"(frame)
                      : "memory");
-    };
-    auto load_rows = [&](uint32_t at, int tile, const uint8_t* base, const uint32_t (&off)[kLoads]) {
-        const int tok0 = tile * kTileTokens + half_off;
-        const uint8_t* frame =
-            base + static_cast<uint64_t>(trow[min(tok0 >> p.tpb_shift, last_blk)]) * p.block_stride;
-        at += 8u * wave * kRow + static_cast<uint32_t>((uintptr_t)lds);
-        if (tok0 + 15 <= last_tok) {
-            frame += static_cast<uint64_t>(tok0 & (p.tpb - 1)) * p.token_stride;
-#pragma unroll
-            for (int i = 0; i < kLoads; ++i) direct_load(at + 1024u * i, off[i], frame);
-        } else {
-#pragma unroll
-            for (int i = 0; i < kLoads; ++i) {
-                const int lr = (8 * wave + kLoadRows * i + lane / kChunks) & 15;
-                const uint32_t in = static_cast<uint32_t>(min(tok0 + lr, last_tok)) & (p.tpb - 1);
-                direct_load(at + 1024u * i, off[i] + (in - static_cast<uint32_t>(lr)) * tstride, frame);
-            }
+        if constexpr (kLoads == 2) {
+            asm volatile("s_add_u32 m0, %0, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                         :
+                         : "s"(at), "v"(off[kLoads - 1]), "s"(frame)
+                         : "memory", "scc");
         }
     };
-    auto load_k = [&](int slot, int tile) { load_rows(slot * kTileBytes, tile, kbase, off_k); };
-    auto load_v = [&](int slot, int tile) { load_rows((kKRing + slot) * kTileBytes, tile, kbase + kv_gap, off_v); };
+    auto load_k = [&](int tile, const uint8_t* frame) {
+        load_rows(lds_rows + (tile & (kRing - 1)) * kTileBytes, frame, off_k);
+    };
+    auto load_v = [&](int tile, const uint8_t* frame) {
+        load_rows(lds_rows + (kRing + (tile & (kRing - 1))) * kTileBytes, frame + kv_gap, off_v);
+    };
+    // Before the loads of a tile: its offsets if it reaches the last half.
+    // (They stay: later tiles load that half again.)
+    auto end_offsets = [&](int tile, uint32_t (&off)[kLoads], bool v) {
+        if (tile * kTileTokens + half_off >= last_half) offsets(off, v, last_tok - last_half);
+    };
+    // Waits until all but the youngest 2 kLoads direct loads have landed.
+    auto wait_older_loads = [&]() { __builtin_amdgcn_s_waitcnt(0x0070 | (2 * kLoads)); };
     // Fragment addresses: the chunks one lane reads of a tile differ by XOR of
     // constant bits (and rows 8 and 16 further), so one address serves them all.
     const uint32_t k_lane = static_cast<uint32_t>(c * kRow + 16 * (h ^ k_key<kD>(c)));
     const int vi = lane & 15;
     const int vrow = 4 * h + (vi >> 2);
     const uint32_t v_lane = static_cast<uint32_t>(
-        kKRing * kTileBytes + vrow * kRow + 16 * ((2 * ((lane >> 4) & 1) + ((vi & 3) >> 1)) ^ v_key<kD>(vrow)) +
+        kRing * kTileBytes + vrow * kRow + 16 * ((2 * ((lane >> 4) & 1) + ((vi & 3) >> 1)) ^ v_key<kD>(vrow)) +
         8 * (vi & 1));
-    static_assert(kKRing * kTileBytes % 256 == 0 && kTileBytes % 256 == 0, "XOR of chunk bits must not carry");
+    static_assert(kTileBytes % 256 == 0, "XOR of chunk bits must not carry");
     // K operands of k-steps x kQk / 2 .. (x + 1) kQk / 2 - 1.
-    auto read_k = [&](int slot, int x, u32x4 (&kf)[kQk / 2]) {
-        const uint32_t a = k_lane + static_cast<uint32_t>(slot) * kTileBytes;
+    auto read_k = [&](int tile, int x, u32x4 (&kf)[kQk / 2]) {
+        const uint32_t a = k_lane + static_cast<uint32_t>(tile & (kRing - 1)) * kTileBytes;
 #pragma unroll
         for (int i = 0; i < kQk / 2; ++i) {
             kf[i] = *(const __attribute__((address_space(3))) u32x4*)(lds + (a ^ (32u * (i + x * kQk / 2))));
         }
     };
     // V operands of row blocks x kHalf .. (x + 1) kHalf - 1, both k-steps.
-    auto read_v = [&](int slot, int x, u32x4 (&vf)[kHalf][2]) {
-        const uint32_t a = v_lane + static_cast<uint32_t>(slot) * kTileBytes;
+    auto read_v = [&](int tile, int x, u32x4 (&vf)[kHalf][2]) {
+        const uint32_t a = v_lane + static_cast<uint32_t>(tile & (kRing - 1)) * kTileBytes;
 #pragma unroll
         for (int n = 0; n < kHalf; ++n)
 #pragma unroll
@@ -293,7 +320,7 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_mfma(DecodeGeometr
     const int t_diag = (pmin + 1) / kTileTokens;  // first tile that needs masks
     const float lazy_raw = kLazy / p.scale_log2;
     floatx16 o[kPv];
-    float lsum;
+    float lsum, m_run;
 
     // One pass over the item's tiles. `careful` (a second pass, taken when the
     // first left a non-finite output) multiplies the masked tiles' V column by
@@ -384,39 +411,67 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_mfma(DecodeGeometr
         floatx16 sa, sb;
         Weights wa, wb;
         u32x4 va[kHalf][2];  // first half of the V operands the next PV takes
-        // A direct load has landed in LDS once vmcnt counts it done: each wave
-        // waits for all of its loads before the barrier that hands the tiles
-        // to the other waves.
-        load_k(0, 0);
-        load_v(0, 0);
-        if (ntiles > 1) load_k(1, 1);
+        // Loads run two steps ahead: step t issues K(t + 3) and V(t + 2) (past
+        // the end the last tile again, into slots nothing reads any more, so
+        // that the count of loads in flight stays the same) and at its end
+        // waits for those of step t - 1 only. (A lone workgroup's step was as
+        // long as one load's latency, 0.75 us, with loads one step ahead.) A
+        // direct load has landed in LDS once vmcnt counts it done: each wave
+        // waits for its own before the barrier that hands the tiles to the
+        // other waves.
+        const uint8_t* frame_v = frame_of(t0, block_of(t0));  // of the tile whose V goes next; its K went a step before
+        const uint8_t* frame_k = frame_of(t0 + 1, block_of(t0 + 1));
+        int blk = block_of(t0 + 2);
+        offsets(off_k, false, 15);
+        offsets(off_v, true, 15);
+        end_offsets(t0, off_k, false);
+        end_offsets(t0, off_v, true);
+        load_k(t0, frame_v);
+        load_v(t0, frame_v);
+        end_offsets(t0 + 1, off_k, false);
+        load_k(t0 + 1, frame_k);
+        // The query loads end here too: left open, the compiler waits for them
+        // (and with them for every tile load) in each step.
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
+        frame_v = frame_k;
+        frame_k = frame_of(t0 + 2, blk);
+        blk = block_of(t0 + 3);
+        end_offsets(t0 + 2, off_k, false);
+        load_k(t0 + 2, frame_k);
+        end_offsets(t0 + 1, off_v, true);
+        load_v(t0 + 1, frame_v);
         if (active) {
             u32x4 k0[kQk / 2], k1[kQk / 2];
-            read_k(0, 0, k0);
-            read_k(0, 1, k1);
+            read_k(t0, 0, k0);
+            read_k(t0, 1, k1);
             qk(k0, 0, sa);
             qk(k1, 1, sa);
-            if (t_diag == 0) mask(sa, 0);
+            if (t_diag <= t0) mask(sa, t0);
             lm = lane_max(sa);
         }
-        __syncthreads();
-        int vslot = 0;  // ring slot of V(t)
         // Step t: the softmax of tile t (s -> w), with QK of tile t + 1 (-> s2)
         // and PV of tile t - 1 (w0) around it: none of the three depends on
         // another, so the matrix products run beside the vector work.
         auto step = [&](int t, const floatx16& s, Weights& w, floatx16& s2, const Weights& w0, auto first, auto masked) {
             constexpr bool kFirst = decltype(first)::value;
             constexpr bool kMasked = decltype(masked)::value;
-            const int vprev = vslot == 0 ? kVRing - 1 : vslot - 1;
-            const int vnext = vslot == kVRing - 1 ? 0 : vslot + 1;
-            load_v(vnext, t + 1);
-            if (t + 2 < ntiles) load_k(t & 1, t + 2);
+            end_offsets(t + 3, off_k, false);
+            end_offsets(t + 2, off_v, true);
+            // Issued among the matrix products (see below): on their own the
+            // address steps hold a lone wave up for a fifth of its step.
+            auto load_ahead = [&]() {
+                frame_v = frame_k;
+                frame_k = frame_of(t + 3, blk);
+                load_k(t + 3, frame_k);
+                load_v(t + 2, frame_v);
+                blk = block_of(t + 4);
+            };
+            if (!active) load_ahead();
             if (active) {
                 raise();
                 u32x4 k0[kQk / 2], k1[kQk / 2], vb[kHalf][2];
-                read_k((t + 1) & 1, 0, k0);
+                read_k(t + 1, 0, k0);
                 if constexpr (!kFirst) {
                     if (kMasked && careful) {
                         pv_careful(va, 0, w0, t - 1);
@@ -424,9 +479,10 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_mfma(DecodeGeometr
                         pv(va, 0, w0);
                     }
                 }
-                read_k((t + 1) & 1, 1, k1);
+                read_k(t + 1, 1, k1);
+                load_ahead();
                 qk(k0, 0, s2);
-                if constexpr (!kFirst) read_v(vprev, 1, vb);
+                if constexpr (!kFirst) read_v(t - 1, 1, vb);
                 qk(k1, 1, s2);
                 lsum += prefill_weights<kF16>(s, p.scale_log2, bias, w.hi, w.lo);
                 if constexpr (!kFirst) {
@@ -436,34 +492,33 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_mfma(DecodeGeometr
                         pv(vb, 1, w0);
                     }
                 }
-                read_v(vslot, 0, va);
+                read_v(t, 0, va);
                 if constexpr (kMasked) mask(s2, t + 1);
                 lm = lane_max(s2);
             }
-            vslot = vnext;
-            __builtin_amdgcn_s_waitcnt(0);
+            wait_older_loads();
             __syncthreads();
         };
-        int t = 0;
-        if (ntiles > 1) {
-            step(0, sa, wa, sb, wa, std::true_type{}, std::true_type{});
+        int t = t0;
+        if (t + 1 < t1) {
+            step(t, sa, wa, sb, wa, std::true_type{}, std::true_type{});
             sa = sb;
-            for (t = 1; t + 2 < min(t_diag, ntiles); t += 2) {
+            for (++t; t + 2 < min(t_diag, t1); t += 2) {
                 step(t, sa, wb, sb, wa, std::false_type{}, std::false_type{});
                 step(t + 1, sb, wa, sa, wb, std::false_type{}, std::false_type{});
             }
-            for (; t < ntiles - 1; ++t) {
+            for (; t < t1 - 1; ++t) {
                 step(t, sa, wb, sb, wa, std::false_type{}, std::true_type{});
                 sa = sb;
                 wa = wb;
             }
         }
-        // Tile t = ntiles - 1: PV of the tile before, its softmax and its own PV.
+        // Tile t = t1 - 1: PV of the tile before, its softmax and its own PV.
         if (active) {
             raise();
             u32x4 vb[kHalf][2];
-            if (t > 0) {
-                read_v(vslot == 0 ? kVRing - 1 : vslot - 1, 1, vb);
+            if (t > t0) {
+                read_v(t - 1, 1, vb);
                 if (careful) {
                     pv_careful(va, 0, wa, t - 1);
                     pv_careful(vb, 1, wa, t - 1);
@@ -474,8 +529,8 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_mfma(DecodeGeometr
             }
             rescale();
             lsum += prefill_weights<kF16>(sa, p.scale_log2, bias, wa.hi, wa.lo);
-            read_v(vslot, 0, va);
-            read_v(vslot, 1, vb);
+            read_v(t, 0, va);
+            read_v(t, 1, vb);
             if (careful) {
                 pv_careful(va, 0, wa, t);
                 pv_careful(vb, 1, wa, t);
@@ -486,9 +541,11 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_mfma(DecodeGeometr
             const auto both =
                 __builtin_amdgcn_permlane32_swap(__float_as_uint(lsum), __float_as_uint(lsum), false, false);
             lsum = __uint_as_float(both[0]) + __uint_as_float(both[1]);
+            m_run = thr == -INFINITY ? -INFINITY : kBias - bias;
         }
     };
     run(false);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last loads land before LDS is used again
     float nonfinite = 0.f;
     if (active) {
 #pragma unroll
@@ -502,8 +559,79 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_mfma(DecodeGeometr
     int bad = 0;
 #pragma unroll
     for (int w = 0; w < kPrefillWaves; ++w) bad |= sm_bad[w];
-    if (__builtin_amdgcn_readfirstlane(bad) != 0) run(true);
+    if (__builtin_amdgcn_readfirstlane(bad) != 0) {
+        run(true);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
 
+    if (nparts > 1) {
+        // The pieces' protocol is the persistent decode's: agent-scope stores,
+        // each wave's wait for them, a barrier, one increment per piece; the
+        // completing workgroup reads the slots with agent-scope loads, in piece
+        // order, so the sum does not depend on who came last.
+        const int slot0 = itp->slot0;
+        if (active) {
+            const uint64_t at = static_cast<uint64_t>(itp->slot) * kPrefillWaves + wave;
+            if (h == 0) {
+                const uint64_t ml = static_cast<uint64_t>(__float_as_uint(lsum)) << 32 | __float_as_uint(m_run);
+                __hip_atomic_store(parts.ml + at * 32 + c, ml, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            uint64_t* acc = parts.acc + at * kPv * 8 * 64 + lane;
+#pragma unroll
+            for (int n = 0; n < kPv; ++n)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const uint64_t x = static_cast<uint64_t>(__float_as_uint(o[n][2 * k + 1])) << 32 |
+                                       __float_as_uint(o[n][2 * k]);
+                    __hip_atomic_store(acc + (n * 8 + k) * 64, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const int done = __hip_atomic_fetch_add(parts.counters + slot0, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            sm_bad[0] = done == nparts - 1;
+            if (done == nparts - 1) {
+                __hip_atomic_store(parts.counters + slot0, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        __syncthreads();
+        if (__builtin_amdgcn_readfirstlane(sm_bad[0]) == 0 || !active) return;
+        const uint64_t first = static_cast<uint64_t>(slot0) * kPrefillWaves + wave;
+        float m_all = -INFINITY;
+        for (int i = 0; i < nparts; ++i) {
+            const uint64_t ml = __hip_atomic_load(parts.ml + (first + i * kPrefillWaves) * 32 + c, __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT);
+            m_all = fmaxf(m_all, __uint_as_float(static_cast<uint32_t>(ml)));
+        }
+        lsum = 0.f;
+#pragma unroll
+        for (int n = 0; n < kPv; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[n][r] = 0.f;
+        for (int i = 0; i < nparts; ++i) {
+            const uint64_t at = first + i * kPrefillWaves;
+            const uint64_t ml = __hip_atomic_load(parts.ml + at * 32 + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const uint64_t* acc = parts.acc + at * kPv * 8 * 64 + lane;
+            uint64_t x[kPv][8];
+#pragma unroll
+            for (int n = 0; n < kPv; ++n)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    x[n][k] = __hip_atomic_load(acc + (n * 8 + k) * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            // A piece whose tokens a row does not see has m = -inf, l = 0, O = 0.
+            const float f = fast_exp2(__uint_as_float(static_cast<uint32_t>(ml)) - m_all);
+            lsum += __uint_as_float(static_cast<uint32_t>(ml >> 32)) * f;
+#pragma unroll
+            for (int n = 0; n < kPv; ++n)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    o[n][2 * k] += __uint_as_float(static_cast<uint32_t>(x[n][k])) * f;
+                    o[n][2 * k + 1] += __uint_as_float(static_cast<uint32_t>(x[n][k] >> 32)) * f;
+                }
+        }
+    }
     if (r0 + 32 * wave + c >= nrows) return;
     // C register r of PV block n in lane (c, h) is O[column c][dim 32n +
     // (r % 4) + 8 (r / 4) + 4h]: four contiguous outputs per r / 4, stored as
@@ -544,24 +672,24 @@ bool prefill_mfma_supported(const DecodeGeometry& g, uint32_t kv_dtype, uintptr_
     const bool aligned = (g.block_stride % 16 == 0) && (g.k_off % 16 == 0) && (g.v_off % 16 == 0) &&
                          (g.token_stride % 16 == 0) && (g.head_stride % 16 == 0) && (kv_base_addr % 16 == 0) &&
                          (query_addr % 16 == 0) && (out_addr % 16 == 0);
-    // A lane's offset inside a 16-token half is kept in 32 bits.
+    // A lane's offset inside a block and the frame stride are kept in 32 bits.
     return (kv_dtype == QVP_DTYPE_BF16 || kv_dtype == QVP_DTYPE_F16) && (g.head_dim == 128 || g.head_dim == 64) &&
-           pow2 && g.tpb >= 16 && aligned && g.token_stride * g.tpb <= 0x7fffffffu;
+           pow2 && g.tpb >= 16 && aligned && g.token_stride * g.tpb <= 0x7fffffffu && g.block_stride <= 0xffffffffu;
 }
 
 template <bool kF16, int kD>
-void launch_prefill(const DecodeGeometry& g, const PrefillItem* items, uint32_t count, uint32_t out_dtype, void* out,
-                    hipStream_t s) {
+void launch_prefill(const DecodeGeometry& g, const PrefillItem* items, uint32_t count, const PrefillParts& parts,
+                    uint32_t out_dtype, void* out, hipStream_t s) {
     const dim3 grid(count), block(kPrefillThreads);
     switch (out_dtype) {
         case QVP_DTYPE_F32:
-            hipLaunchKernelGGL((prefill_mfma<kF16, kD, float>), grid, block, 0, s, g, items, out);
+            hipLaunchKernelGGL((prefill_mfma<kF16, kD, float>), grid, block, 0, s, g, items, parts, out);
             break;
         case QVP_DTYPE_BF16:
-            hipLaunchKernelGGL((prefill_mfma<kF16, kD, uint16_t>), grid, block, 0, s, g, items, out);
+            hipLaunchKernelGGL((prefill_mfma<kF16, kD, uint16_t>), grid, block, 0, s, g, items, parts, out);
             break;
         default:
-            hipLaunchKernelGGL((prefill_mfma<kF16, kD, _Float16>), grid, block, 0, s, g, items, out);
+            hipLaunchKernelGGL((prefill_mfma<kF16, kD, _Float16>), grid, block, 0, s, g, items, parts, out);
             break;
     }
 }
@@ -579,9 +707,109 @@ void destroy_prefill_plan(qvp_prefill_plan& p) {
     if (p.staging != nullptr) (void)hipHostFree(p.staging);
     if (p.staging_done != nullptr) (void)hipEventDestroy(p.staging_done);
     if (p.device != nullptr) (void)hipFree(p.device);
+    if (p.parts != nullptr) (void)hipFree(p.parts);
     if (p.virt != nullptr) (void)qvp_batch_destroy(p.virt);
+    destroy_reader(p.reader);
     p = qvp_prefill_plan{};
 }
+
+namespace {
+
+// Bytes of one workspace slot (head_dim 128), and the most slots a plan uses
+// (64 MB): beyond them items stay whole.
+constexpr size_t kPartBytes = kPrefillRows * (128 + 2) * sizeof(float);
+constexpr uint32_t kMaxParts = 1024;
+
+// How many pieces an item of nt tiles is cut into when a CU's share of the
+// launch is `share` tiles: two workgroups share a CU and a lone one runs its
+// tiles faster, so only items past 1.25 shares end late. Every piece costs its
+// merger about three tiles' time (64 KB through the workspace), which makes
+// sqrt(nt / 3) pieces the best for an item alone on the chip. (One item of 126
+// tiles alone: 80.6 us whole, 28.8 us in 6 pieces; 63 tiles: 42.8 and 23.1 us;
+// cutting to T / 512 tiles whatever the share put 4 prompts of up to 1024
+// tokens at 46.5 us against 38.3 us whole, the workspace traffic being 75 MB.)
+uint32_t piece_count(uint32_t nt, double share) {
+    if (nt <= 1.25 * share) return 1;
+    const uint32_t most = static_cast<uint32_t>(std::sqrt(nt / 3.0));
+    return std::max<uint32_t>(1, std::min(most, static_cast<uint32_t>(std::ceil(nt / std::max(share, 1.0)))));
+}
+
+// The work list of one prefill, longest items first, so that the short ones
+// fill the end. When all workgroups are resident at once (two per CU) none
+// waits for another: the second half then goes shortest first, which puts the
+// longest and the shortest on one CU.
+std::vector<PrefillItem> plan_items(const std::vector<int32_t>& lens, const uint32_t* q_start, uint32_t group,
+                                    uint32_t kv_heads, uint32_t cus, uint32_t* num_parts) {
+    std::vector<PrefillItem> whole;
+    uint64_t tiles = 0;
+    uint32_t longest = 0;
+    int32_t row = 0;
+    for (size_t sq = 0; sq < lens.size(); ++sq) {
+        const int32_t start = static_cast<int32_t>(q_start[sq]);
+        const int32_t nrows = (lens[sq] - start) * static_cast<int32_t>(group);
+        for (int32_t r0 = 0; r0 < nrows; r0 += kPrefillRows) {
+            const int32_t last = start + (std::min(r0 + kPrefillRows, nrows) - 1) / static_cast<int32_t>(group);
+            const int32_t nt = last / kTileTokens + 1;
+            tiles += static_cast<uint64_t>(nt) * kv_heads;
+            longest = std::max(longest, static_cast<uint32_t>(nt));
+            for (uint32_t kv = 0; kv < kv_heads; ++kv) {
+                whole.push_back(PrefillItem{static_cast<int32_t>(sq), static_cast<int32_t>(kv), start, r0, nrows, row, 0,
+                                            nt, -1, -1, 1, 0});
+            }
+        }
+        row += lens[sq] - start;
+    }
+    const double share = static_cast<double>(tiles) / cus;
+    uint32_t used = 0;
+    std::vector<PrefillItem> items;
+    items.reserve(whole.size() + kMaxParts);
+    for (const PrefillItem& it : whole) {
+        const uint32_t nt = static_cast<uint32_t>(it.t1);
+        const uint32_t n = piece_count(nt, share);
+        if (n < 2 || used + n > kMaxParts) {
+            items.push_back(it);
+            continue;
+        }
+        for (uint32_t i = 0; i < n; ++i) {
+            PrefillItem piece = it;
+            piece.t0 = static_cast<int32_t>(nt * i / n);
+            piece.t1 = static_cast<int32_t>(nt * (i + 1) / n);
+            piece.slot = static_cast<int32_t>(used + i);
+            piece.slot0 = static_cast<int32_t>(used);
+            piece.nparts = static_cast<int32_t>(n);
+            items.push_back(piece);
+        }
+        used += n;
+    }
+    *num_parts = used;
+    // Longest first: a counting sort on the tile count (stable).
+    std::vector<uint32_t> at(longest + 2, 0);
+    for (const PrefillItem& it : items) ++at[longest - static_cast<uint32_t>(it.t1 - it.t0) + 1];
+    for (size_t i = 1; i < at.size(); ++i) at[i] += at[i - 1];
+    std::vector<PrefillItem> sorted(items.size());
+    for (const PrefillItem& it : items) sorted[at[longest - static_cast<uint32_t>(it.t1 - it.t0)]++] = it;
+    if (sorted.size() > cus && sorted.size() <= 2 * static_cast<size_t>(cus)) {
+        std::reverse(sorted.begin() + cus, sorted.end());
+    }
+    return sorted;
+}
+
+// Grows a device buffer that earlier prefills on `s` or on the plan's last
+// stream may still read.
+int grow(void** ptr, size_t* cap, size_t need, const qvp_reader& reader, hipStream_t s) {
+    if (*ptr != nullptr) {
+        QVP_HIP(hipStreamSynchronize(s));
+        if (reader.pending && reader.stream != s) QVP_HIP(hipStreamSynchronize(reader.stream));
+        QVP_HIP(hipFree(*ptr));
+    }
+    *ptr = nullptr;
+    *cap = 0;
+    QVP_HIP(hipMalloc(ptr, need));
+    *cap = need;
+    return QVP_OK;
+}
+
+}  // namespace
 
 }  // namespace qvp
 
@@ -712,74 +940,95 @@ extern "C" int qvp_paged_prefill(const qvp_prefill_args* a, void* stream) {
         return flush();
     }
 
-    // Work items, longest context first.
-    const uint64_t G = g.group;
-    std::vector<qvp::PrefillItem> items;
-    uint32_t row = 0;
-    for (uint32_t sq = 0; sq < v.num_seqs; ++sq) {
-        const uint32_t start = a->q_start[sq];
-        const uint32_t fresh = static_cast<uint32_t>(lens[sq]) - start;
-        if (fresh * G > 0x7fffffffu - qvp::kPrefillRows) return fail(QVP_ERR_INVALID_ARGUMENT, "too many new tokens");
-        const uint32_t nrows = static_cast<uint32_t>(fresh * G);
-        for (uint32_t r0 = 0; r0 < nrows; r0 += qvp::kPrefillRows) {
-            for (uint32_t kv = 0; kv < a->num_kv_heads; ++kv) {
-                items.push_back(qvp::PrefillItem{static_cast<int32_t>(sq), static_cast<int32_t>(kv),
-                                                 static_cast<int32_t>(start), static_cast<int32_t>(r0),
-                                                 static_cast<int32_t>(nrows), static_cast<int32_t>(row)});
-            }
+    // (Made and uploaded on every call, four prompts of 2048 tokens took 57 us
+    // more alone than back to back; 28 us in the first call of a pack now.)
+    // The plan depends on the pack (its context lengths), the first new
+    // positions and the grouping: a call with the same ones (the next layer)
+    // finds it on the device. Another stream than the last call's makes it
+    // anew, after that call's kernel.
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    QVP_HIP(hipStreamIsCapturing(s, &capture));
+    const bool capturing = capture != hipStreamCaptureStatusNone;
+    if (!capturing) QVP_TRY(qvp::wait_for_reader(plan.reader, s));
+    const bool current = plan.valid && plan.generation == batch->generation && plan.stream == s &&
+                         plan.group == g.group && plan.num_kv_heads == g.num_kv_heads &&
+                         plan.q_start.size() == v.num_seqs &&
+                         std::equal(plan.q_start.begin(), plan.q_start.end(), a->q_start);
+    if (!current) {
+        for (uint32_t sq = 0; sq < v.num_seqs; ++sq) {
+            const uint64_t rows = static_cast<uint64_t>(static_cast<uint32_t>(lens[sq]) - a->q_start[sq]) * g.group;
+            if (rows > 0x7fffffffu - qvp::kPrefillRows) return fail(QVP_ERR_INVALID_ARGUMENT, "too many new tokens");
         }
-        row += fresh;
-    }
-    const auto last_token = [G](const qvp::PrefillItem& x) {
-        return x.start + (std::min(x.r0 + qvp::kPrefillRows, x.nrows) - 1) / static_cast<int32_t>(G);
-    };
-    std::stable_sort(items.begin(), items.end(), [&](const qvp::PrefillItem& x, const qvp::PrefillItem& y) {
-        return last_token(x) > last_token(y);
-    });
-    if (items.size() > 0x7fffffffu) return fail(QVP_ERR_INVALID_ARGUMENT, "too many prefill items");
-    const size_t ints = items.size() * (sizeof(qvp::PrefillItem) / sizeof(int32_t));
-    // Host-side reuse of pinned staging only: no system-scope release.
-    if (plan.staging_done == nullptr) {
-        QVP_HIP(hipEventCreateWithFlags(&plan.staging_done, hipEventDisableTiming | hipEventDisableSystemFence));
-    }
-    if (plan.staging_pending) {
-        QVP_HIP(hipEventSynchronize(plan.staging_done));
-        plan.staging_pending = false;
-    }
-    if (plan.staging_cap < ints) {
-        if (plan.staging != nullptr) QVP_HIP(hipHostFree(plan.staging));
-        plan.staging = nullptr;
-        plan.staging_cap = 0;
-        QVP_HIP(hipHostMalloc(reinterpret_cast<void**>(&plan.staging), ints * sizeof(int32_t), hipHostMallocCoherent));
-        plan.staging_cap = ints;
-    }
-    if (plan.device_cap < ints) {
-        // The device list may still be read by an earlier prefill on this batch.
-        if (plan.device != nullptr) {
-            QVP_HIP(hipStreamSynchronize(s));
-            QVP_HIP(hipFree(plan.device));
+        int dev = 0, cus = 0;
+        QVP_HIP(hipGetDevice(&dev));
+        QVP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        uint32_t parts = 0;
+        const std::vector<qvp::PrefillItem> items = qvp::plan_items(
+            lens, a->q_start, g.group, g.num_kv_heads, static_cast<uint32_t>(std::max(cus, 1)), &parts);
+        if (items.size() > 0x7fffffffu) return fail(QVP_ERR_INVALID_ARGUMENT, "too many prefill items");
+        plan.valid = false;
+        const size_t bytes = items.size() * sizeof(qvp::PrefillItem);
+        // Host-side reuse of pinned staging only: no system-scope release.
+        if (plan.staging_done == nullptr) {
+            QVP_HIP(hipEventCreateWithFlags(&plan.staging_done, hipEventDisableTiming | hipEventDisableSystemFence));
         }
-        plan.device = nullptr;
-        plan.device_cap = 0;
-        QVP_HIP(hipMalloc(reinterpret_cast<void**>(&plan.device), ints * sizeof(int32_t)));
-        plan.device_cap = ints;
+        if (plan.staging_pending) {
+            QVP_HIP(hipEventSynchronize(plan.staging_done));
+            plan.staging_pending = false;
+        }
+        if (plan.staging_cap < bytes) {
+            if (plan.staging != nullptr) QVP_HIP(hipHostFree(plan.staging));
+            plan.staging = nullptr;
+            plan.staging_cap = 0;
+            QVP_HIP(hipHostMalloc(&plan.staging, bytes, hipHostMallocCoherent));
+            plan.staging_cap = bytes;
+        }
+        if (plan.device_cap < bytes) QVP_TRY(qvp::grow(&plan.device, &plan.device_cap, bytes, plan.reader, s));
+        const size_t counter_bytes = qvp::round_up(parts * sizeof(int32_t), 256);
+        if (parts > 0 && plan.parts_cap < counter_bytes + parts * qvp::kPartBytes) {
+            const size_t need = counter_bytes + parts * qvp::kPartBytes;
+            QVP_TRY(qvp::grow(&plan.parts, &plan.parts_cap, need, plan.reader, s));
+            plan.parts_clean = false;
+        }
+        // Every launch leaves its counters at zero, but their number moves the
+        // results behind them, which earlier plans wrote.
+        if (parts > 0 && (!plan.parts_clean || plan.num_parts != parts)) {
+            QVP_TRY(qvp_fill_bytes(plan.parts, 0, counter_bytes, s));
+            plan.parts_clean = true;
+        }
+        if (parts > 0) plan.num_parts = parts;
+        std::memcpy(plan.staging, items.data(), bytes);
+        QVP_TRY(qvp::pull_from_pinned(plan.device, plan.staging, bytes, s));
+        QVP_HIP(hipEventRecord(plan.staging_done, s));
+        plan.staging_pending = true;
+        plan.num_items = static_cast<uint32_t>(items.size());
+        plan.stream = s;
+        plan.generation = batch->generation;
+        plan.group = g.group;
+        plan.num_kv_heads = g.num_kv_heads;
+        plan.q_start.assign(a->q_start, a->q_start + v.num_seqs);
+        plan.valid = true;
     }
-    std::memcpy(plan.staging, items.data(), ints * sizeof(int32_t));
-    QVP_TRY(qvp::pull_from_pinned(plan.device, plan.staging, ints * sizeof(int32_t), s));
-    QVP_HIP(hipEventRecord(plan.staging_done, s));
-    plan.staging_pending = true;
 
-    const auto* dev_items = reinterpret_cast<const qvp::PrefillItem*>(plan.device);
-    const uint32_t count = static_cast<uint32_t>(items.size());
+    const auto* dev_items = static_cast<const qvp::PrefillItem*>(plan.device);
+    const uint32_t count = plan.num_items;
+    qvp::PrefillParts parts{};
+    if (plan.parts != nullptr) {
+        uint8_t* base = static_cast<uint8_t*>(plan.parts);
+        parts.counters = reinterpret_cast<int32_t*>(base);
+        parts.ml = reinterpret_cast<uint64_t*>(base + qvp::round_up(plan.num_parts * sizeof(int32_t), 256));
+        parts.acc = parts.ml + static_cast<uint64_t>(plan.num_parts) * qvp::kPrefillRows;
+    }
     const bool f16 = a->kv_dtype == QVP_DTYPE_F16;
     if (g.head_dim == 128) {
-        f16 ? qvp::launch_prefill<true, 128>(g, dev_items, count, a->out_dtype, a->out, s)
-            : qvp::launch_prefill<false, 128>(g, dev_items, count, a->out_dtype, a->out, s);
+        f16 ? qvp::launch_prefill<true, 128>(g, dev_items, count, parts, a->out_dtype, a->out, s)
+            : qvp::launch_prefill<false, 128>(g, dev_items, count, parts, a->out_dtype, a->out, s);
     } else {
-        f16 ? qvp::launch_prefill<true, 64>(g, dev_items, count, a->out_dtype, a->out, s)
-            : qvp::launch_prefill<false, 64>(g, dev_items, count, a->out_dtype, a->out, s);
+        f16 ? qvp::launch_prefill<true, 64>(g, dev_items, count, parts, a->out_dtype, a->out, s)
+            : qvp::launch_prefill<false, 64>(g, dev_items, count, parts, a->out_dtype, a->out, s);
     }
     QVP_HIP(hipGetLastError());
+    QVP_TRY(qvp::note_reader(plan.reader, s, s));
     // The kernel reads the packed block tables: a later pack into this slot
     // from another stream waits for it.
     return qvp::note_reader(batch->readers[batch->current], s, batch->upload_stream[batch->current]);

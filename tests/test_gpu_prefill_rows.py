@@ -68,3 +68,36 @@ def test_later_tokens_that_are_not_finite_do_not_reach_earlier_rows(d, dtype):
     assert_close_bf16(got[:40], ref32[:40], "rows before the infinite token")
     # (A weight is two products here, so a seen infinity may come out as NaN.)
     assert not np.isfinite(got[40:]).any() and not np.isfinite(ref32[40:]).any()
+
+
+def test_split_items_and_kept_plans():
+    # Few rows behind long contexts are cut into pieces that one workgroup
+    # merges; the plan (and the pieces' counters) is kept between calls with the
+    # same first positions and made anew for others, on either stream. Every
+    # call must give the bits of its first one.
+    print("case: prefill pieces, kept and changed plans, two streams", flush=True)
+    lens = [4100, 777, 33]
+    w, q = _inputs(lens, [0, 0, 0], 14, 2, 128, qvp.DTYPE_BF16)
+    starts = {"tail": [4091, 770, 32], "last": [4099, 776, 30], "long": [3800, 0, 0]}
+    stream = qvp.Stream()
+    seen = {}
+    run = None
+    for name in ("tail", "last", "tail", "long", "tail", "last"):
+        q_start = starts[name]
+        rows = np.concatenate([q[sum(lens[:b]) + a: sum(lens[:b + 1])] for b, a in enumerate(q_start)])
+        if name not in seen:
+            got, _, ref32, (run, args, out, dq) = _run(w, q_start, qvp.DTYPE_F32, queries=rows)
+            assert_close_bf16(got, ref32, name)
+            seen[name] = (got, args, out, dq, run)
+    # One batch for all three, packed once.
+    _, _, _, _, run = seen["tail"]
+    for on in (None, stream, None):
+        for name in ("tail", "last", "tail", "tail", "long", "last"):
+            got, args, out, _, _ = seen[name]
+            args.batch = run.batch.handle
+            out.fill(0xFF)
+            qvp.synchronize()
+            qvp.paged_prefill(args, on)
+            qvp.synchronize()
+            again = out.download(np.float32, got.shape)
+            assert np.array_equal(again.view(np.uint32), got.view(np.uint32)), f"{name} on {on}"
