@@ -357,13 +357,16 @@ typedef enum qvp_decode_kernel {
     QVP_DECODE_MFMA = 1,        /* persistent bf16 MFMA kernel, cost-balanced tile ranges */
     QVP_DECODE_F32_GROUPED = 2, /* fp32 MFMA kernel over split_tokens partitions + merge */
     QVP_DECODE_GENERIC = 3,     /* VALU kernel per query head over split_tokens partitions + merge */
-    QVP_DECODE_GROUPED = 4,     /* VALU kernel per kv head (GQA group folded) over split_tokens partitions + merge */
+    QVP_DECODE_GROUPED = 4,     /* kernel per kv head (GQA group folded) over split_tokens partitions + merge:
+                                   matrix cores for bf16/fp16 at head_dim 96 and 256, vector ALUs otherwise */
     QVP_DECODE_SPLIT_MFMA = 5   /* bf16/fp16 MFMA kernel per kv head at head_dim 64 over split_tokens partitions + merge */
 } qvp_decode_kernel;
 
 typedef struct qvp_decode_plan {
     uint32_t kernel;            /* qvp_decode_kernel */
-    uint32_t workgroups;        /* workgroups of the decode kernel */
+    uint32_t workgroups;        /* MFMA: workgroups of the decode kernel; split kernels: units of a
+                                   partition and a kv head (generic: a query head). A unit may be
+                                   spread over several workgroups, or share one with its neighbours */
     uint32_t pieces;            /* MFMA: (sequence, kv-head group, tile range) pieces;
                                    split kernels: token partitions */
     uint32_t slots;             /* partial results merged through the workspace */
@@ -420,10 +423,10 @@ typedef struct qvp_prefill_args {
 /* Validates everything on the host (the decode's rules, plus q_start[b] <
  * seq_lens[b]), then enqueues the prefill on `stream`. bf16 and fp16 caches
  * with head_dim 128 or 64, a positive scale, power-of-two tokens_per_block >=
- * 16, and query, out, kv_base and the strides in bytes all multiples of 16 run
- * the MFMA prefill kernel (any query group); everything else runs the decode
- * kernels over one virtual sequence per new position (packed in chunks of at
- * most 2^20 block ids, decoded in order on `stream`). */
+ * 16, query groups of at most 16, and query, out, kv_base and the strides in
+ * bytes all multiples of 16 run the MFMA prefill kernel; everything else runs
+ * the decode kernels over one virtual sequence per new position (packed in
+ * chunks of at most 2^20 block ids, decoded in order on `stream`). */
 int qvp_paged_prefill(const qvp_prefill_args* args, void* stream);
 
 /* ------------------------------------------------------------------------ */

@@ -174,12 +174,19 @@ struct qvp_batch {
     std::vector<uint32_t> ids_scratch;
     std::vector<uint32_t> cu_scratch;
     qvp_packed_view view{};
+    // Per sequence kSplitCounterHeads completion counters in the packed buffer,
+    // zero between launches (NULL: none packed).
+    int32_t* split_counters{nullptr};
     qvp_decode_plan last_plan{};       // what the last decode on this pack ran (reset by qvp_pack)
     qvp_schedule sched{};
     qvp_prefill_plan prefill{};
 };
 
 namespace qvp {
+// Batches of up to this many sequences carry counters for the split kernels'
+// in-launch merge, for up to this many kv heads.
+constexpr uint32_t kSplitCounterSeqs = 1024;
+constexpr uint32_t kSplitCounterHeads = 16;
 // A pack's upload taken over by a decode launch: 16-byte words src -> dst
 // (src is the device mapping of the pinned staging), then `tail` 4-byte
 // words after them.

@@ -61,7 +61,9 @@ template <> __device__ inline _Float16 from_float<_Float16>(float v) { return st
 int launch_generic_decode(const DecodeGeometry& g, const qvp_packed_view& v, uint32_t kv_dtype,
                           uint32_t out_dtype, void* out, void* workspace, hipEvent_t split_event,
                           hipStream_t stream);
-uint64_t generic_workspace_bytes(const qvp_packed_view& v, uint32_t hq, uint32_t d);
+// Workspace of a split kernel's partial results: (m, l) and O per split, part of
+// it and query head.
+uint64_t generic_workspace_bytes(const qvp_packed_view& v, uint32_t hq, uint32_t d, uint32_t parts = 1);
 // GQA-folded split decode (groups of 1 .. 16, any element type, head_dim a
 // multiple of four up to 1024 with rows aligned to four elements, its LDS
 // within 64 KiB): one workgroup per (split, kv head), the generic workspace
@@ -69,18 +71,20 @@ uint64_t generic_workspace_bytes(const qvp_packed_view& v, uint32_t hq, uint32_t
 bool grouped_supported(const DecodeGeometry& g, uint32_t kv_dtype, uint32_t split_tokens);
 int launch_grouped_decode(const DecodeGeometry& g, const qvp_packed_view& v, uint32_t kv_dtype, uint32_t out_dtype,
                           void* out, void* workspace, hipEvent_t split_event, hipStream_t stream);
-// Combines the per-split (m, l, O) of the generic workspace layout into the
-// output (one workgroup per (sequence, query head)).
-int launch_merge_splits(const DecodeGeometry& g, const qvp_packed_view& v, uint32_t out_dtype, void* out,
-                        const float* ws_ml, const float* ws_acc, hipStream_t stream);
+// Combines the (m, l, O) of the generic workspace layout into the output. A split holds `parts` slots, one per
+// split_tokens / parts tokens; those past a sequence's end are not read.
+int launch_merge_splits(const DecodeGeometry& g, const qvp_packed_view& v, uint32_t parts, uint32_t out_dtype,
+                        void* out, const float* ws_ml, const float* ws_acc, hipStream_t stream);
 
 // fp32 caches, head_dim 128 or 64, GQA group <= 16, power-of-two tpb >= 16, splits a
 // multiple of 16 tokens: the fp32 MFMA kernel, one workgroup per (split, kv
-// head), in the generic workspace layout. Returns a qvp_status.
+// head), each split cut into `parts` parts, in the generic workspace layout.
+// Counters as in decode_split16.h. Returns a qvp_status.
 bool f32_grouped_supported(const DecodeGeometry& g, uint32_t kv_dtype, uint32_t split_tokens, uintptr_t query_addr,
                            uintptr_t kv_base_addr);
-int launch_f32_grouped_decode(const DecodeGeometry& g, const qvp_packed_view& v, uint32_t out_dtype, void* out,
-                              void* workspace, hipEvent_t split_event, hipStream_t stream);
+int launch_f32_grouped_decode(const DecodeGeometry& g, const qvp_packed_view& v, uint32_t parts, int32_t* counters,
+                              uint32_t out_dtype, void* out, void* workspace, hipEvent_t split_event,
+                              hipStream_t stream);
 
 // Vector tiles of the persistent kernel take query groups up to this size;
 // the automatic choice uses them for groups up to kVectorTilesUpToGroup (0:

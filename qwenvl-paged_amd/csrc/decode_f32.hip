@@ -18,6 +18,7 @@
 // LDS and write the split's (m, l, O) in the generic kernel's workspace
 // layout; the generic split merge produces the output.
 #include "mfma_tile.h"
+#include "split_merge.h"
 
 namespace qvp {
 namespace {
@@ -30,8 +31,11 @@ struct F32SplitArgs {
     const int32_t* split_seq;
     const int32_t* split_start;
     uint32_t split_tokens;
-    float* ws_ml;   // [num_splits][Hq][2]: running max (base 2), running sum
-    float* ws_acc;  // [num_splits][Hq][D]
+    uint32_t parts_shift;  // log2 of the ranges per split
+    uint32_t part_tokens;  // split_tokens / parts, a multiple of 16
+    SplitOutput so;
+    float* ws_ml;   // [num_splits * parts][Hq][2]: running max (base 2), running sum
+    float* ws_acc;  // [num_splits * parts][Hq][D]
 };
 
 // One 16-token block of K and V for head_dim kD (128 or 64).
@@ -62,19 +66,24 @@ __global__ __launch_bounds__(kF32Threads, 2) void decode_f32_grouped(DecodeGeome
     constexpr int kV = kD / 64;      // V loads per lane and token
     __shared__ float sm_m[kF32Waves][16];
     __shared__ float sm_l[kF32Waves][16];
-    __shared__ float sm_o[kF32Waves][16][kRowPad];
+    static_assert(kF32Waves * 16 * kRowPad >= kMergeLds && kF32Threads == kMergeWg, "the merge takes over the waves' LDS");
+    __shared__ __attribute__((aligned(16))) float sm_o[kF32Waves][16][kRowPad];
+    __shared__ int sm_last;
 
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
     const int c = lane & 15;
     const int j = lane >> 4;
     const int G = static_cast<int>(p.group);
-    const int split = static_cast<int>(blockIdx.x / p.num_kv_heads);
-    const int g = static_cast<int>(blockIdx.x - split * p.num_kv_heads);
+    const int part = static_cast<int>(blockIdx.x / p.num_kv_heads);
+    const int g = static_cast<int>(blockIdx.x - part * p.num_kv_heads);
+    const int split = part >> sa.parts_shift;
     const int b = as_const(sa.split_seq)[split];
-    const int start = as_const(sa.split_start)[split];
+    const int start = as_const(sa.split_start)[split] +
+                      (part - (split << sa.parts_shift)) * static_cast<int>(sa.part_tokens);
     const int ctx = as_const(p.seq_lens)[b];
-    const int end = min(start + static_cast<int>(sa.split_tokens), ctx);
+    const int end = min(start + static_cast<int>(sa.part_tokens), ctx);
+    if (start >= end) return;  // a range past the context: it has no slot
     const int nblk = (end - start + kF32Block - 1) / kF32Block;
     const auto* row = as_const(p.tables) + static_cast<uint64_t>(b) * p.max_nb;
     const uint32_t tmask = p.tpb - 1;
@@ -176,27 +185,26 @@ __global__ __launch_bounds__(kF32Threads, 2) void decode_f32_grouped(DecodeGeome
 #pragma unroll
         for (int n = 0; n < kK; ++n) sm_o[wave][c][(kD / 4) * j + (kD / 16) * r + n] = o[n][r];
     __syncthreads();
-    const uint64_t head0 = static_cast<uint64_t>(split) * p.num_q_heads + static_cast<uint64_t>(g) * G;
-    for (int e = threadIdx.x; e < G * kD; e += kF32Threads) {
-        const int hc = e / kD;
-        const int dd = e - hc * kD;
-        float mmax = sm_m[0][hc];
+    const int split_tokens = static_cast<int>(sa.split_tokens);
+    const SlotRange slots = slots_of(split - as_const(sa.split_start)[split] / split_tokens, ctx, split_tokens,
+                                     static_cast<int>(sa.parts_shift));
+    auto value = [&](int hc, int d4, float& m, float& l) {
+        m = sm_m[0][hc];
 #pragma unroll
-        for (int w = 1; w < kF32Waves; ++w) mmax = fmaxf(mmax, sm_m[w][hc]);
-        float acc = 0.f;
-        float lsum = 0.f;
+        for (int w = 1; w < kF32Waves; ++w) m = fmaxf(m, sm_m[w][hc]);
+        floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+        l = 0.f;
 #pragma unroll
         for (int w = 0; w < kF32Waves; ++w) {
-            const float f = fast_exp2(sm_m[w][hc] - mmax);
-            acc += sm_o[w][hc][dd] * f;
-            lsum += sm_l[w][hc] * f;
+            const float f = fast_exp2(sm_m[w][hc] - m);
+            acc += *reinterpret_cast<const floatx4*>(&sm_o[w][hc][d4]) * f;
+            l += sm_l[w][hc] * f;
         }
-        sa.ws_acc[(head0 + hc) * kD + dd] = acc;
-        if (dd == 0) {
-            sa.ws_ml[(head0 + hc) * 2 + 0] = mmax;
-            sa.ws_ml[(head0 + hc) * 2 + 1] = lsum;
-        }
-    }
+        return acc;
+    };
+    finish_part<kD>(sa.so, sa.ws_ml, sa.ws_acc, slots, static_cast<uint64_t>(part), static_cast<uint32_t>(b),
+                    static_cast<uint32_t>(g * G), G, p.num_q_heads,
+                    static_cast<uint32_t>(b) * p.num_kv_heads + static_cast<uint32_t>(g), value, &sm_o[0][0][0], &sm_last);
 }
 
 }  // namespace
@@ -211,16 +219,20 @@ bool f32_grouped_supported(const DecodeGeometry& g, uint32_t kv_dtype, uint32_t 
            pow2 && g.tpb >= 16 && split_tokens % kF32Block == 0 && aligned;
 }
 
-int launch_f32_grouped_decode(const DecodeGeometry& g, const qvp_packed_view& v, uint32_t out_dtype, void* out,
-                              void* workspace, hipEvent_t split_event, hipStream_t stream) {
-    const uint64_t heads = static_cast<uint64_t>(v.num_splits) * g.num_q_heads;
+int launch_f32_grouped_decode(const DecodeGeometry& g, const qvp_packed_view& v, uint32_t parts, int32_t* counters,
+                              uint32_t out_dtype, void* out, void* workspace, hipEvent_t split_event,
+                              hipStream_t stream) {
+    const uint64_t heads = static_cast<uint64_t>(v.num_splits) * parts * g.num_q_heads;
     F32SplitArgs sa{};
     sa.split_seq = v.split_seq;
     sa.split_start = v.split_start;
     sa.split_tokens = v.split_tokens;
+    while ((1u << sa.parts_shift) < parts) ++sa.parts_shift;
+    sa.part_tokens = v.split_tokens / parts;
+    sa.so = SplitOutput{out, out_dtype, counters};
     sa.ws_ml = static_cast<float*>(workspace);
     sa.ws_acc = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + round_up(heads * 2 * sizeof(float), 256));
-    const uint64_t groups = static_cast<uint64_t>(v.num_splits) * g.num_kv_heads;
+    const uint64_t groups = static_cast<uint64_t>(v.num_splits) * parts * g.num_kv_heads;
     if (groups > 0x7fffffffu) return fail(QVP_ERR_INVALID_ARGUMENT, "too many (split, kv head) pairs");
     if (g.head_dim == 64) {
         hipLaunchKernelGGL(decode_f32_grouped<64>, dim3(static_cast<unsigned>(groups)), dim3(kF32Threads), 0, stream, g,
@@ -231,7 +243,8 @@ int launch_f32_grouped_decode(const DecodeGeometry& g, const qvp_packed_view& v,
     }
     QVP_HIP(hipGetLastError());
     if (split_event != nullptr) QVP_HIP(hipEventRecord(split_event, stream));
-    return launch_merge_splits(g, v, out_dtype, out, sa.ws_ml, sa.ws_acc, stream);
+    if (counters != nullptr) return QVP_OK;
+    return launch_merge_splits(g, v, parts, out_dtype, out, sa.ws_ml, sa.ws_acc, stream);
 }
 
 }  // namespace qvp

@@ -7,6 +7,7 @@
 // combines the splits of each sequence. It serves fp32/fp16 caches and shapes
 // the MFMA kernel does not cover.
 #include "decode_common.h"
+#include "split_merge.h"
 
 #include <algorithm>
 
@@ -106,64 +107,100 @@ __global__ __launch_bounds__(kGenericThreads) void decode_generic(DecodeGeometry
     }
 }
 
-// out = sum_s acc_s 2^(m_s - M) / sum_s l_s 2^(m_s - M) per (sequence, head).
-// Up to kMergeThreads splits: thread s reads split s's (m, l) once, the
-// maximum and the weighted sum are workgroup reductions and the splits'
-// factors sit in LDS for the accumulation pass (one round trip for the
-// (m, l) pairs instead of two dependent loops over them).
-constexpr int kMergeThreads = 128;
+// Up to kMergeSlots slots per sequence, groups up to kMergeRows and a head_dim
+// of a multiple of four: one workgroup per (sequence, kv head), with the
+// arithmetic of the in-launch merge.
+__global__ __launch_bounds__(kMergeWg) void merge_groups(SplitOutput so, const float* ws_ml, const float* ws_acc,
+                                                         const int32_t* __restrict__ cu_splits,
+                                                         const int32_t* __restrict__ seq_lens, uint32_t num_q_heads,
+                                                         uint32_t num_kv_heads, uint32_t head_dim,
+                                                         uint32_t split_tokens, uint32_t parts_shift) {
+    __shared__ float lds[kMergeLds];
+    const uint32_t b = blockIdx.x / num_kv_heads;
+    const uint32_t g = blockIdx.x - b * num_kv_heads;
+    const int group = static_cast<int>(num_q_heads / num_kv_heads);
+    const SlotRange slots = slots_of(cu_splits[b], seq_lens[b], static_cast<int>(split_tokens),
+                                     static_cast<int>(parts_shift));
+    merge_rows(so, ws_ml, ws_acc, slots, b, g * group, group, num_q_heads, static_cast<int>(head_dim), lds);
+}
 
-template <typename OutT>
+// Any number of slots, group and head_dim, one workgroup per (sequence, head):
+// out = sum_s acc_s 2^(m_s - M) / sum_s l_s 2^(m_s - M) over its slots s. The
+// slots' factors sit in LDS a workgroup's worth at a time, and the accumulators
+// are read as kVec floats per thread by as many threads as there are columns,
+// times the row groups that fit beside them (a group takes every groups-th
+// slot; the groups are added in order).
+constexpr int kMergeThreads = 256;
+
+template <typename OutT, int kVec>
 __global__ __launch_bounds__(kMergeThreads) void merge_splits(const float* __restrict__ ws_ml,
                                                              const float* __restrict__ ws_acc,
                                                              const int32_t* __restrict__ cu_splits,
+                                                             const int32_t* __restrict__ seq_lens,
                                                              OutT* __restrict__ out, uint32_t num_q_heads,
-                                                             uint32_t head_dim) {
+                                                             uint32_t head_dim, uint32_t split_tokens, uint32_t parts_shift) {
+    typedef float vec __attribute__((ext_vector_type(kVec)));
     __shared__ float f_s[kMergeThreads];
     __shared__ float red[kMergeThreads / 64];
+    __shared__ __attribute__((aligned(16))) float part_s[kMergeThreads * kVec];
     const uint32_t b = blockIdx.x / num_q_heads;
     const uint32_t h = blockIdx.x - b * num_q_heads;
-    const int s0 = cu_splits[b];
-    const int s1 = cu_splits[b + 1];
-    const int ns = s1 - s0;
-    if (ns <= kMergeThreads) {
-        const int t = static_cast<int>(threadIdx.x);
-        float m = -INFINITY;
-        float l = 0.f;
-        if (t < ns) {
-            const uint64_t idx = static_cast<uint64_t>(s0 + t) * num_q_heads + h;
-            m = ws_ml[idx * 2];
-            l = ws_ml[idx * 2 + 1];
-        }
-        const float mmax = block_reduce_max(m, red);
-        const float f = t < ns ? fast_exp2(m - mmax) : 0.f;
-        f_s[t] = f;
-        const float lsum = block_reduce_sum(l * f, red);  // also orders the f_s writes before the reads below
-        OutT* o = out + (static_cast<uint64_t>(b) * num_q_heads + h) * head_dim;
-        for (uint32_t d = threadIdx.x; d < head_dim; d += blockDim.x) {
-            float acc = 0.f;
-            for (int x = 0; x < ns; ++x) {
-                acc += ws_acc[(static_cast<uint64_t>(s0 + x) * num_q_heads + h) * head_dim + d] * f_s[x];
-            }
-            o[d] = from_float<OutT>(acc / lsum);
-        }
-        return;
+    const int t = static_cast<int>(threadIdx.x);
+    const SlotRange slots = slots_of(cu_splits[b], seq_lens[b], static_cast<int>(split_tokens),
+                                     static_cast<int>(parts_shift));
+    const int ns = slots.count;
+    const uint64_t slot0 = slots.first;
+    auto ml_at = [&](int s) {
+        return *reinterpret_cast<const float2*>(ws_ml + ((slot0 + s) * num_q_heads + h) * 2);
+    };
+
+    float2 ml{-INFINITY, 0.f};
+    if (t < ns) ml = ml_at(t);
+    float mmax = ml.x;
+    for (int s = t + kMergeThreads; s < ns; s += kMergeThreads) mmax = fmaxf(mmax, ml_at(s).x);
+    mmax = block_reduce_max(mmax, red);
+    float f = t < ns ? fast_exp2(ml.x - mmax) : 0.f;
+    float l = ml.y * f;
+    for (int s = t + kMergeThreads; s < ns; s += kMergeThreads) {
+        const float2 x = ml_at(s);
+        l += x.y * fast_exp2(x.x - mmax);
     }
-    float mmax = -INFINITY;
-    for (int s = s0; s < s1; ++s) mmax = fmaxf(mmax, ws_ml[(static_cast<uint64_t>(s) * num_q_heads + h) * 2]);
-    float lsum = 0.f;
-    for (int s = s0; s < s1; ++s) {
-        const uint64_t idx = static_cast<uint64_t>(s) * num_q_heads + h;
-        lsum += ws_ml[idx * 2 + 1] * fast_exp2(ws_ml[idx * 2] - mmax);
-    }
+    f_s[t] = f;
+    const float lsum = block_reduce_sum(l, red);  // also orders the f_s writes before the reads below
+
+    const int cols = static_cast<int>(head_dim) / kVec;
+    const int groups = cols >= kMergeThreads ? 1 : kMergeThreads / cols;
+    const int grp = cols >= kMergeThreads ? 0 : t / cols;
     OutT* o = out + (static_cast<uint64_t>(b) * num_q_heads + h) * head_dim;
-    for (uint32_t d = threadIdx.x; d < head_dim; d += blockDim.x) {
-        float acc = 0.f;
-        for (int s = s0; s < s1; ++s) {
-            const uint64_t idx = static_cast<uint64_t>(s) * num_q_heads + h;
-            acc += ws_acc[idx * head_dim + d] * fast_exp2(ws_ml[idx * 2] - mmax);
+    for (int c0 = 0; c0 < cols; c0 += kMergeThreads) {
+        const int col = cols >= kMergeThreads ? c0 + t : t - grp * cols;
+        const bool mine = grp < groups && col < cols;
+        vec acc = {};
+        for (int base = 0; base < ns; base += kMergeThreads) {
+            if (ns > kMergeThreads) {
+                // More slots than threads: the factors of this stretch of them.
+                __syncthreads();
+                f_s[t] = base + t < ns ? fast_exp2(ml_at(base + t).x - mmax) : 0.f;
+                __syncthreads();
+            }
+            if (!mine) continue;
+            const float* a = ws_acc + ((slot0 + base) * num_q_heads + h) * head_dim + col * kVec;
+            const uint64_t step = static_cast<uint64_t>(num_q_heads) * head_dim;
+            const int n = min(ns - base, kMergeThreads);
+#pragma unroll 8
+            for (int x = grp; x < n; x += groups) acc += *reinterpret_cast<const vec*>(a + x * step) * f_s[x];
         }
-        o[d] = from_float<OutT>(acc / lsum);
+        if (groups > 1) {
+            *reinterpret_cast<vec*>(part_s + t * kVec) = acc;
+            __syncthreads();
+            if (grp == 0) {
+                for (int k = 1; k < groups; ++k) acc += *reinterpret_cast<const vec*>(part_s + (k * cols + col) * kVec);
+            }
+        }
+        if (mine && grp == 0) {
+#pragma unroll
+            for (int e = 0; e < kVec; ++e) o[col * kVec + e] = from_float<OutT>(acc[e] / lsum);
+        }
     }
 }
 
@@ -435,11 +472,11 @@ int launch_grouped_decode(const DecodeGeometry& g, const qvp_packed_view& v, uin
     }
     QVP_HIP(hipGetLastError());
     if (split_event != nullptr) QVP_HIP(hipEventRecord(split_event, stream));
-    return launch_merge_splits(g, v, out_dtype, out, sa.ws_ml, sa.ws_acc, stream);
+    return launch_merge_splits(g, v, 1, out_dtype, out, sa.ws_ml, sa.ws_acc, stream);
 }
 
-uint64_t generic_workspace_bytes(const qvp_packed_view& v, uint32_t hq, uint32_t d) {
-    const uint64_t heads = static_cast<uint64_t>(v.num_splits) * hq;
+uint64_t generic_workspace_bytes(const qvp_packed_view& v, uint32_t hq, uint32_t d, uint32_t parts) {
+    const uint64_t heads = static_cast<uint64_t>(v.num_splits) * parts * hq;
     return round_up(heads * 2 * sizeof(float), 256) + round_up(heads * d * sizeof(float), 256);
 }
 
@@ -472,25 +509,44 @@ int launch_generic_decode(const DecodeGeometry& g, const qvp_packed_view& v, uin
     QVP_HIP(hipGetLastError());
     if (split_event != nullptr) QVP_HIP(hipEventRecord(split_event, stream));
 
-    return launch_merge_splits(g, v, out_dtype, out, sa.ws_ml, sa.ws_acc, stream);
+    return launch_merge_splits(g, v, 1, out_dtype, out, sa.ws_ml, sa.ws_acc, stream);
 }
 
-int launch_merge_splits(const DecodeGeometry& g, const qvp_packed_view& v, uint32_t out_dtype, void* out,
-                        const float* ws_ml, const float* ws_acc, hipStream_t stream) {
-    const dim3 mgrid(v.num_seqs * g.num_q_heads);
+namespace {
+
+template <typename OutT>
+void launch_merge_for(const DecodeGeometry& g, const qvp_packed_view& v, uint32_t shift, void* out, const float* ws_ml,
+                      const float* ws_acc, hipStream_t stream) {
+    const dim3 grid(v.num_seqs * g.num_q_heads);
+    OutT* o = static_cast<OutT*>(out);
+    if (g.head_dim % 4 == 0) {
+        hipLaunchKernelGGL((merge_splits<OutT, 4>), grid, dim3(kMergeThreads), 0, stream, ws_ml, ws_acc, v.cu_splits,
+                           v.seq_lens, o, g.num_q_heads, g.head_dim, v.split_tokens, shift);
+    } else {
+        hipLaunchKernelGGL((merge_splits<OutT, 1>), grid, dim3(kMergeThreads), 0, stream, ws_ml, ws_acc, v.cu_splits,
+                           v.seq_lens, o, g.num_q_heads, g.head_dim, v.split_tokens, shift);
+    }
+}
+
+}  // namespace
+
+int launch_merge_splits(const DecodeGeometry& g, const qvp_packed_view& v, uint32_t parts, uint32_t out_dtype,
+                        void* out, const float* ws_ml, const float* ws_acc, hipStream_t stream) {
+    const uint32_t part_tokens = v.split_tokens / parts;
+    uint32_t shift = 0;
+    while ((1u << shift) < parts) ++shift;
+    if (g.head_dim % 4 == 0 && g.group <= static_cast<uint32_t>(kMergeRows) &&
+        (v.max_seq_len + part_tokens - 1) / part_tokens <= static_cast<uint32_t>(kMergeSlots)) {
+        hipLaunchKernelGGL(merge_groups, dim3(v.num_seqs * g.num_kv_heads), dim3(kMergeWg), 0, stream,
+                           SplitOutput{out, out_dtype, nullptr}, ws_ml, ws_acc, v.cu_splits, v.seq_lens,
+                           g.num_q_heads, g.num_kv_heads, g.head_dim, v.split_tokens, shift);
+        QVP_HIP(hipGetLastError());
+        return QVP_OK;
+    }
     switch (out_dtype) {
-        case QVP_DTYPE_F32:
-            hipLaunchKernelGGL(merge_splits<float>, mgrid, dim3(kMergeThreads), 0, stream, ws_ml, ws_acc, v.cu_splits,
-                               static_cast<float*>(out), g.num_q_heads, g.head_dim);
-            break;
-        case QVP_DTYPE_BF16:
-            hipLaunchKernelGGL(merge_splits<uint16_t>, mgrid, dim3(kMergeThreads), 0, stream, ws_ml, ws_acc, v.cu_splits,
-                               static_cast<uint16_t*>(out), g.num_q_heads, g.head_dim);
-            break;
-        default:
-            hipLaunchKernelGGL(merge_splits<_Float16>, mgrid, dim3(kMergeThreads), 0, stream, ws_ml, ws_acc, v.cu_splits,
-                               static_cast<_Float16*>(out), g.num_q_heads, g.head_dim);
-            break;
+        case QVP_DTYPE_F32: launch_merge_for<float>(g, v, shift, out, ws_ml, ws_acc, stream); break;
+        case QVP_DTYPE_BF16: launch_merge_for<uint16_t>(g, v, shift, out, ws_ml, ws_acc, stream); break;
+        default: launch_merge_for<_Float16>(g, v, shift, out, ws_ml, ws_acc, stream); break;
     }
     QVP_HIP(hipGetLastError());
     return QVP_OK;

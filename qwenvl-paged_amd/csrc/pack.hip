@@ -287,7 +287,12 @@ int pack_impl(qvp_batch* batch, uint32_t num_seqs, const uint32_t* block_ids, co
             QVP_TRY(qvp::mfma_plan_schedule(batch->sched, sin, g));
         }
     }
-    const size_t total = lay.total + (with_schedule ? batch->sched.total : 0);
+    // Zeroed completion counters of the split kernels' in-launch merge, unless
+    // the decode is known to be another (or the batch large: 64 bytes a sequence).
+    const size_t counters = with_schedule || num_seqs > qvp::kSplitCounterSeqs
+                                ? 0
+                                : align_ints(static_cast<size_t>(num_seqs) * qvp::kSplitCounterHeads);
+    const size_t total = lay.total + (with_schedule ? batch->sched.total : counters);
 
     // A pack still waiting for its upload (qvp_pack_ahead) is superseded.
     if (batch->upload_pending[0] || batch->upload_pending[1]) {
@@ -351,7 +356,11 @@ int pack_impl(qvp_batch* batch, uint32_t num_seqs, const uint32_t* block_ids, co
     }
     cu_seqlens[num_seqs] = token_acc;
     cu_splits[num_seqs] = split_acc;
-    if (with_schedule) qvp::mfma_write_schedule(batch->sched, sin, h + lay.total);
+    if (with_schedule) {
+        qvp::mfma_write_schedule(batch->sched, sin, h + lay.total);
+    } else {
+        std::fill_n(h + lay.total, counters, 0);
+    }
 
     // The pack before last (same slot) may still be read by a decode on
     // another stream; one upload then carries the arrays and the schedule
@@ -385,6 +394,7 @@ int pack_impl(qvp_batch* batch, uint32_t num_seqs, const uint32_t* block_ids, co
         batch->sched.in_pack_buffer = true;
         batch->sched.valid = true;
     }
+    batch->split_counters = counters > 0 ? d + lay.total : nullptr;
     qvp_packed_view& v = batch->view;
     v.block_tables = d + lay.tables;
     v.seq_lens = d + lay.seq_lens;

@@ -8,7 +8,7 @@
 // (:73-89). Only then is anything enqueued, so a refused call leaves `out`
 // untouched. bf16, fp16 and fp32 caches with head_dim 128 run the persistent
 // MFMA kernel (decode_mfma.hip); other shapes run a split kernel: the fp32
-// MFMA one (decode_f32.hip), the 16-bit MFMA one for head_dim 64
+// MFMA one (decode_f32.hip), the 16-bit MFMA one for head_dim 64, 96 and 256
 // (decode_split16.hip), the GQA-folded one for groups up to 16 with
 // four-element rows, or the per-query-head generic one (both in
 // decode_generic.hip).
@@ -102,6 +102,37 @@ uint64_t mfma_bound_bytes(const qvp_packed_view& v, uint32_t hq, uint32_t d) {
     return qvp::round_up(rows * 2 * sizeof(float), 256) + qvp::round_up(rows * d * sizeof(float), 256);
 }
 
+// Parts (a power of two) the matrix-core split kernels cut each split into.
+// One workgroup merges a (sequence, kv head)'s parts, in the launch while they
+// are at most kMaxFusedParts.
+//
+// Rows of up to 256 bytes (head_dim 64 in fp32, 64 and 96 in 16 bits): parts are
+// halved, down to 64 tokens, until half the CUs have a workgroup; more of them
+// only add merging. Event-timed at 512 / 256 / 128 / 64 tokens a part, fp32
+// head_dim 64: 4 sequences of up to 509 tokens, 2 kv heads (8 workgroups with
+// whole splits), 10.1 / 9.2 / 8.0 / 7.4 us; up to 1850 tokens, 4 kv heads (48)
+// 14.5 / 11.5 / 11.8 / 16.1; 16 kv heads (192) 15.2 / 15.9 / 17.7 / 23.9. Longer
+// rows (head_dim 256) keep a workgroup's four waves busy with 128 tokens, and
+// large batches want four workgroups per CU: bf16, 2 sequences of 1000 tokens, 8
+// kv heads, 19.5 / 14.8 / 13.3 / 16.2; 32 sequences of 512 .. 4096, 4 kv heads
+// (620), 65.4 / 63.0 / 71.0 (232 us on the vector kernel).
+constexpr uint32_t kMaxFusedParts = 16;
+uint32_t most_parts(const qvp_packed_view& v, uint32_t parts) {
+    const uint32_t part_tokens = v.split_tokens / parts;
+    return (v.max_seq_len + part_tokens - 1) / part_tokens;
+}
+uint32_t split_parts(const qvp_packed_view& v, uint32_t kv_heads, uint32_t row_bytes) {
+    const uint64_t workgroups = row_bytes > 256 ? 1024 : 128;
+    const uint32_t least = row_bytes > 256 ? 128 : 64;
+    uint32_t parts = 1;
+    while (static_cast<uint64_t>(v.num_splits) * kv_heads * parts < workgroups &&
+           v.split_tokens % (2 * parts * 32) == 0 && v.split_tokens / (2 * parts) >= least &&
+           most_parts(v, 2 * parts) <= kMaxFusedParts) {
+        parts *= 2;
+    }
+    return parts;
+}
+
 }  // namespace
 
 namespace qvp {
@@ -189,7 +220,8 @@ int qvp_decode_workspace_bytes(const qvp_batch* batch, uint32_t num_query_heads,
     QVP_TRY(qvp_batch_view(batch, &v));
     // Shared-prefix slots come on top of the persistent kernel's own bound.
     const uint64_t prefix_rows = qvp::mfma_prefix_slot_bound(batch) * num_query_heads;
-    *bytes = std::max(qvp::generic_workspace_bytes(v, num_query_heads, head_dim),
+    *bytes = std::max(qvp::generic_workspace_bytes(v, num_query_heads, head_dim,
+                                                         split_parts(v, 1, head_dim > 96 ? 512 : 256)),
                       mfma_bound_bytes(v, num_query_heads, head_dim) +
                           qvp::round_up(prefix_rows * 2 * sizeof(float), 256) +
                           qvp::round_up(prefix_rows * head_dim * sizeof(float), 256));
@@ -235,11 +267,24 @@ int decode_impl(const qvp_decode_args* a, void* stream, bool no_alloc) {
         return fail(QVP_ERR_INVALID_ARGUMENT,
                     "the batch's qvp_pack_ahead upload is still pending: enqueue it (qvp_batch_upload) before capture");
     }
+    const bool f32 = !mfma && qvp::f32_grouped_supported(g, a->kv_dtype, v.split_tokens,
+                                                         reinterpret_cast<uintptr_t>(a->query),
+                                                         reinterpret_cast<uintptr_t>(a->kv_base));
+    const bool s16 = !mfma && !f32 &&
+                     qvp::split16_supported(g, a->kv_dtype, v.split_tokens, reinterpret_cast<uintptr_t>(a->query));
+    uint32_t parts = 1;
     if (mfma) {
         QVP_TRY(qvp::mfma_prepare_schedule(batch, g, s, !no_alloc));
         need = qvp::mfma_workspace_bytes(batch, g.group, g.head_dim);
     } else {
-        need = qvp::generic_workspace_bytes(v, a->num_query_heads, a->head_dim);
+        if (f32 || s16) {
+            parts = split_parts(v, a->num_kv_heads,
+                                a->head_dim * static_cast<uint32_t>(qvp::dtype_size(a->kv_dtype)));
+        }
+        // Finer parts only where the given workspace holds their results.
+        const uint64_t room = no_alloc ? kScratchBytes : ws != nullptr ? a->workspace_bytes : UINT64_MAX;
+        while (parts > 1 && qvp::generic_workspace_bytes(v, a->num_query_heads, a->head_dim, parts) > room) parts /= 2;
+        need = qvp::generic_workspace_bytes(v, a->num_query_heads, a->head_dim, parts);
     }
     if (no_alloc) {
         if (need > kScratchBytes) {
@@ -277,20 +322,28 @@ int decode_impl(const qvp_decode_args* a, void* stream, bool no_alloc) {
         plan.shared_prefix_groups = sc.prefix_groups;
         plan.shared_prefix_items = sc.num_prefix_items;
     } else {
-        const bool f32 = qvp::f32_grouped_supported(g, a->kv_dtype, v.split_tokens,
-                                                    reinterpret_cast<uintptr_t>(a->query),
-                                                    reinterpret_cast<uintptr_t>(a->kv_base));
-        const bool s16 = !f32 && qvp::split16_supported(g, a->kv_dtype, v.split_tokens,
-                                                        reinterpret_cast<uintptr_t>(a->query));
         const bool grouped = !f32 && !s16 && qvp::grouped_supported(g, a->kv_dtype, v.split_tokens);
-        status = f32       ? qvp::launch_f32_grouped_decode(g, v, a->out_dtype, a->out, ws, ev, s)
-                 : s16     ? qvp::launch_split16_decode(g, v, a->kv_dtype, a->out_dtype, a->out, ws, ev, s)
+        // The in-launch merge counts in the batch's own counters: decodes that
+        // could overlap another of the batch (a captured one, or one on another
+        // stream than the last) leave the merge to its launch.
+        const qvp_reader& last = batch->readers[batch->current];
+        // A launch that fills the chip several times over in fp32 ends its
+        // workgroups sooner without it (64 sequences: 73.9 against 75.1 us).
+        int32_t* counters = nullptr;
+        const uint64_t units = static_cast<uint64_t>(v.num_splits) * parts * a->num_kv_heads;
+        if ((s16 || (f32 && units <= 512)) && !capturing && a->num_kv_heads <= qvp::kSplitCounterHeads &&
+            most_parts(v, parts) <= kMaxFusedParts && !(last.pending && last.stream != s)) {
+            counters = batch->split_counters;
+        }
+        status = f32       ? qvp::launch_f32_grouped_decode(g, v, parts, counters, a->out_dtype, a->out, ws, ev, s)
+                 : s16     ? qvp::launch_split16_decode(g, v, parts, counters, a->kv_dtype, a->out_dtype, a->out, ws,
+                                                               ev, s)
                  : grouped ? qvp::launch_grouped_decode(g, v, a->kv_dtype, a->out_dtype, a->out, ws, ev, s)
                            : qvp::launch_generic_decode(g, v, a->kv_dtype, a->out_dtype, a->out, ws, ev, s);
-        plan.kernel = f32       ? QVP_DECODE_F32_GROUPED
-                      : s16     ? QVP_DECODE_SPLIT_MFMA
-                      : grouped ? QVP_DECODE_GROUPED
-                                : QVP_DECODE_GENERIC;
+        plan.kernel = f32                        ? QVP_DECODE_F32_GROUPED
+                      : s16 && g.head_dim == 64  ? QVP_DECODE_SPLIT_MFMA
+                      : s16 || grouped           ? QVP_DECODE_GROUPED
+                                                 : QVP_DECODE_GENERIC;
         plan.workgroups = v.num_splits * (f32 || s16 || grouped ? a->num_kv_heads : a->num_query_heads);
         plan.pieces = v.num_splits;
         plan.slots = v.num_splits;

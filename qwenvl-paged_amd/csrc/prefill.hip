@@ -4,11 +4,11 @@
 // PagedAttention.h:43-44; tests/EndToEnd.test.cpp:252-256), so every output
 // row here is the decode of its position.
 //
-// MFMA path (bf16 or fp16 cache, head_dim 128 or 64, power-of-two
-// tokens_per_block >= 16). The rows of (sequence b, kv head g) are its new
+// MFMA path (bf16 or fp16 cache, head_dim 128 or 64, GQA group <= 16,
+// power-of-two tokens_per_block >= 16). The rows of (sequence b, kv head g) are its new
 // positions times the G query heads of g's group, position-major, so row r is
 // head r % G at position q_start + r / G; a work item is 128 consecutive rows
-// (a cut may fall inside a position: every wave is full for any group size).
+// (a cut may fall inside a position: every wave is full for any group).
 // Its workgroup streams the tokens its last row sees in 32-token tiles: each
 // tile is loaded once, straight into LDS, one tile of compute ahead of its
 // use, into a double buffer holding the K and V rows as in the frame (16-byte
@@ -139,8 +139,10 @@ __device__ inline float lane_max(const floatx16& s) {
 }
 
 // P of one tile as the hi and lo B operands of the PV k-steps; returns this
-// lane's sum of its sixteen weights. bf16: hi = P truncated, lo = P - hi
-// rounded to nearest even. (v_dot2_f32_bf16 gives p - hi in one instruction,
+// lane's sum of its sixteen weights. hi and lo = P - hi are both rounded to
+// nearest even: 2^-18 of a weight at most for bf16 (2^-17 with hi truncated, at
+// the same instruction count; no weight is exactly 1 here, as the largest is
+// under a maximum that moves with every tile). (v_dot2_f32_bf16 gives p - hi in one instruction,
 // but holds the matrix core up: beside MFMAs it costs as much as three others.)
 template <bool kF16>
 __device__ inline float prefill_weights(const floatx16& s, float scale_log2, float bias, u32x4 (&hi)[2],
@@ -158,12 +160,11 @@ __device__ inline float prefill_weights(const floatx16& s, float scale_log2, flo
             hi[r / 8][(r / 2) & 3] = __builtin_bit_cast(uint32_t, a);
             lo[r / 8][(r / 2) & 3] = __builtin_bit_cast(uint32_t, b);
         } else {
-            const uint32_t b0 = __float_as_uint(p0);
-            const uint32_t b1 = __float_as_uint(p1);
-            const bf16x2_t b = {static_cast<__bf16>(p0 - __uint_as_float(b0 & 0xffff0000u)),
-                                static_cast<__bf16>(p1 - __uint_as_float(b1 & 0xffff0000u))};
-            // High halves of p0 (low word) and p1 (high word) in one byte permute.
-            hi[r / 8][(r / 2) & 3] = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
+            const bf16x2_t a = {static_cast<__bf16>(p0), static_cast<__bf16>(p1)};
+            const uint32_t x = __builtin_bit_cast(uint32_t, a);
+            const bf16x2_t b = {static_cast<__bf16>(p0 - __uint_as_float(x << 16)),
+                                static_cast<__bf16>(p1 - __uint_as_float(x & 0xffff0000u))};
+            hi[r / 8][(r / 2) & 3] = x;
             lo[r / 8][(r / 2) & 3] = __builtin_bit_cast(uint32_t, b);
         }
     }
@@ -672,9 +673,11 @@ bool prefill_mfma_supported(const DecodeGeometry& g, uint32_t kv_dtype, uintptr_
     const bool aligned = (g.block_stride % 16 == 0) && (g.k_off % 16 == 0) && (g.v_off % 16 == 0) &&
                          (g.token_stride % 16 == 0) && (g.head_stride % 16 == 0) && (kv_base_addr % 16 == 0) &&
                          (query_addr % 16 == 0) && (out_addr % 16 == 0);
-    // A lane's offset inside a block and the frame stride are kept in 32 bits.
+    // Groups above 16 decode on the vector kernel, with fp32 weights, and so
+    // prefill there. A lane's offset inside a block and the frame stride are
+    // kept in 32 bits.
     return (kv_dtype == QVP_DTYPE_BF16 || kv_dtype == QVP_DTYPE_F16) && (g.head_dim == 128 || g.head_dim == 64) &&
-           pow2 && g.tpb >= 16 && aligned && g.token_stride * g.tpb <= 0x7fffffffu && g.block_stride <= 0xffffffffu;
+           g.group >= 1 && g.group <= 16 && pow2 && g.tpb >= 16 && aligned && g.token_stride * g.tpb <= 0x7fffffffu && g.block_stride <= 0xffffffffu;
 }
 
 template <bool kF16, int kD>
