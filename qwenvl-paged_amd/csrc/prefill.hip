@@ -142,8 +142,9 @@ __device__ inline float lane_max(const floatx16& s) {
 // lane's sum of its sixteen weights. hi and lo = P - hi are both rounded to
 // nearest even: 2^-18 of a weight at most for bf16 (2^-17 with hi truncated, at
 // the same instruction count; no weight is exactly 1 here, as the largest is
-// under a maximum that moves with every tile). (v_dot2_f32_bf16 gives p - hi in one instruction,
-// but holds the matrix core up: beside MFMAs it costs as much as three others.)
+// under a maximum that moves with every tile). v_dot2_f32_bf16 would give p - hi
+// in one instruction, but holds the matrix core up: beside MFMAs it costs as
+// much as three others.
 template <bool kF16>
 __device__ inline float prefill_weights(const floatx16& s, float scale_log2, float bias, u32x4 (&hi)[2],
                                         u32x4 (&lo)[2]) {

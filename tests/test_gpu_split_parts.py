@@ -99,3 +99,18 @@ def test_weights_keep_24_bits_where_the_vector_kernel_kept_fp32():
         _, ref32 = oracle_decode(w, run.image, run.query)
         err = float(np.abs(got - ref32).max() / np.abs(ref32).max())
         assert err <= 2e-6, f"d={d}: {err:.3e}"
+
+
+@pytest.mark.parametrize("lens,hq,hkv", [([1], 28, 4), ([1501], 28, 4), ([1024, 993], 32, 8), ([2048], 28, 4),
+                                         ([32, 33, 4096], 28, 4), ([16384], 28, 4), ([16385], 28, 4)],
+                         ids=["one token", "one sequence", "8 heads", "full lanes", "uneven", "last even", "first weighted"])
+def test_persistent_decode_with_about_one_tile_per_lane(lens, hq, hkv):
+    # Ranges of equal length while each tile lane has one tile at most (256
+    # workgroups of 8 waves and 4 kv heads: 512 tiles of 32 tokens), in
+    # proportion to the heads' weights beyond: every token counted once.
+    print(f"case: one tile per lane {lens} hq={hq} hkv={hkv}", flush=True)
+    w = W.custom(lens, hq, hkv, 128, num_layers=2, layer=1, seed=len(lens) + lens[-1])
+    run = GpuRun(w)
+    _, ref32 = oracle_decode(w, run.image, run.query)
+    assert_close_bf16(run.decode(out_dtype=qvp.DTYPE_F32), ref32, "fp32 out")
+    assert run.batch.decode_plan()["kernel"] == "mfma"
