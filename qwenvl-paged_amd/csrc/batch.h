@@ -175,8 +175,11 @@ struct qvp_batch {
     std::vector<uint32_t> cu_scratch;
     qvp_packed_view view{};
     // Per sequence kSplitCounterHeads completion counters in the packed buffer,
-    // zero between launches (NULL: none packed).
+    // zero between launches (NULL: none packed), and the stream whose decodes
+    // count in them (the first to do so since the pack).
     int32_t* split_counters{nullptr};
+    bool split_counters_used{false};
+    hipStream_t split_counter_stream{nullptr};
     qvp_decode_plan last_plan{};       // what the last decode on this pack ran (reset by qvp_pack)
     qvp_schedule sched{};
     qvp_prefill_plan prefill{};

@@ -395,6 +395,7 @@ int pack_impl(qvp_batch* batch, uint32_t num_seqs, const uint32_t* block_ids, co
         batch->sched.valid = true;
     }
     batch->split_counters = counters > 0 ? d + lay.total : nullptr;
+    batch->split_counters_used = false;
     qvp_packed_view& v = batch->view;
     v.block_tables = d + lay.tables;
     v.seq_lens = d + lay.seq_lens;

@@ -324,16 +324,19 @@ int decode_impl(const qvp_decode_args* a, void* stream, bool no_alloc) {
     } else {
         const bool grouped = !f32 && !s16 && qvp::grouped_supported(g, a->kv_dtype, v.split_tokens);
         // The in-launch merge counts in the batch's own counters: decodes that
-        // could overlap another of the batch (a captured one, or one on another
-        // stream than the last) leave the merge to its launch.
-        const qvp_reader& last = batch->readers[batch->current];
+        // could overlap another that does (a captured one, or one on another
+        // stream than the first to count in since the pack) leave the merge to
+        // its launch. The stream of the last decode is not enough: after decodes
+        // on streams 1, 2 and 2 the first may still be counting.
         // A launch that fills the chip several times over in fp32 ends its
         // workgroups sooner without it (64 sequences: 73.9 against 75.1 us).
         int32_t* counters = nullptr;
         const uint64_t units = static_cast<uint64_t>(v.num_splits) * parts * a->num_kv_heads;
         if ((s16 || (f32 && units <= 512)) && !capturing && a->num_kv_heads <= qvp::kSplitCounterHeads &&
-            most_parts(v, parts) <= kMaxFusedParts && !(last.pending && last.stream != s)) {
+            most_parts(v, parts) <= kMaxFusedParts && !(batch->split_counters_used && batch->split_counter_stream != s)) {
             counters = batch->split_counters;
+            batch->split_counters_used = true;
+            batch->split_counter_stream = s;
         }
         status = f32       ? qvp::launch_f32_grouped_decode(g, v, parts, counters, a->out_dtype, a->out, ws, ev, s)
                  : s16     ? qvp::launch_split16_decode(g, v, parts, counters, a->kv_dtype, a->out_dtype, a->out, ws,

@@ -101,6 +101,34 @@ def test_weights_keep_24_bits_where_the_vector_kernel_kept_fp32():
         assert err <= 2e-6, f"d={d}: {err:.3e}"
 
 
+def test_decodes_of_one_pack_on_several_streams():
+    # Only one stream's decodes may count in the pack's counters: a decode on
+    # stream A, then two on B, where the second must not take B's turn as the
+    # end of A's. Every result has the bits of the first.
+    print("case: one pack on two streams", flush=True)
+    dtype, hq, hkv, d, tpb = qvp.DTYPE_BF16, 28, 4, 256, 16
+    lens = [4000, 900, 2300, 33] * 4
+    w = W.custom(lens, hq, hkv, d, kv_dtype=dtype, tokens_per_block=tpb, seed=3)
+    run = GpuRun(w)
+    want = run.decode(out_dtype=qvp.DTYPE_F32)
+    streams = [qvp.Stream(), qvp.Stream()]
+    outs = [qvp.DeviceBuffer(want.nbytes) for _ in range(3)]
+    run.batch.pack(w.ids, w.cu_blocks, w.context_lens, tpb, w.num_pool_blocks, 0)
+    qvp.synchronize()
+    spaces = [qvp.DeviceBuffer(run.batch.workspace_bytes(hq, d)) for _ in outs]
+    for k in range(20):
+        for on, out, ws in zip((streams[0], streams[1], streams[1]), outs, spaces):
+            qvp.paged_decode(qvp.decode_args(query=run.q.ptr, out=out.ptr, kv_base=run.pool.base,
+                                             block_stride=run.pool.stride, batch=run.batch, kv_dtype=dtype,
+                                             out_dtype=qvp.DTYPE_F32, layer=w.layer, num_layers=w.num_layers,
+                                             num_query_heads=hq, num_kv_heads=hkv, head_dim=d, tokens_per_block=tpb,
+                                             scale=w.scale, strides=w.strides, workspace=ws.ptr,
+                                             workspace_bytes=ws.nbytes), on)
+        qvp.synchronize()
+        for i, out in enumerate(outs):
+            assert np.array_equal(out.download(np.float32, want.shape), want), f"round {k}, decode {i}"
+
+
 @pytest.mark.parametrize("lens,hq,hkv", [([1], 28, 4), ([1501], 28, 4), ([1024, 993], 32, 8), ([2048], 28, 4),
                                          ([32, 33, 4096], 28, 4), ([16384], 28, 4), ([16385], 28, 4)],
                          ids=["one token", "one sequence", "8 heads", "full lanes", "uneven", "last even", "first weighted"])
