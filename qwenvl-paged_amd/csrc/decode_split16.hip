@@ -101,6 +101,7 @@ __global__ __launch_bounds__(kS16Threads, 2) void decode_split16(DecodeGeometry 
     constexpr int kK = kD / 32;
     constexpr int kN = kD / 16;
     constexpr int kTerms = kF16 || kD == 64 ? 2 : 3;
+    using E = std::conditional_t<kF16, _Float16, uint16_t>;
     constexpr int kRowPad = kD + 4;  // LDS row of one merged output column (floats)
     constexpr int kLds = kS16Waves * 16 * kRowPad;  // floats
     static_assert(kLds >= kMergeLds, "the merge takes over the waves' LDS");
@@ -329,6 +330,30 @@ __global__ __launch_bounds__(kS16Threads, 2) void decode_split16(DecodeGeometry 
             const float f = mw == -INFINITY ? 0.f : fast_exp2(mw - m);
             acc += *reinterpret_cast<const floatx4*>(sm_o + (w * 16 + hc) * kRowPad + d4) * f;
             l += sm_l[w][hc] * f;
+        }
+        if constexpr (kD != 64) {
+            // An infinite value meets a weight's terms one by one, and a zero or
+            // negative lower term makes NaN of it where the whole weight gives
+            // infinity. Such sums are taken again token by token.
+            const bool nan = acc[0] != acc[0] || acc[1] != acc[1] || acc[2] != acc[2] || acc[3] != acc[3];
+            if (nan && m > -INFINITY && m < INFINITY) {
+                const float bias = (kF16 ? kF16WeightLog2 : 0.f) - m;
+                acc = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+                for (int tok = start; tok < end; ++tok) {
+                    const uint8_t* at = kbase + static_cast<uint64_t>(row[tok >> p.tpb_shift]) * p.block_stride +
+                                        (static_cast<uint32_t>(tok) & tmask) * tstride;
+                    const E* k = reinterpret_cast<const E*>(at);
+                    const E* v = reinterpret_cast<const E*>(at + kv_gap) + d4;
+                    const E* q = reinterpret_cast<const E*>(q0) + hc * kD;
+                    float sc = 0.f;
+#pragma unroll 1
+                    for (int x = 0; x < kD; ++x) sc = fmaf(to_float<E>(q[x]), to_float<E>(k[x]), sc);
+                    const float pw = fast_exp2(fmaf(sc, p.scale_log2, bias));
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) acc[x] = fmaf(pw, to_float<E>(v[x]), acc[x]);
+                }
+            }
         }
         return acc;
     };

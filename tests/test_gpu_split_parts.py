@@ -101,6 +101,32 @@ def test_weights_keep_24_bits_where_the_vector_kernel_kept_fp32():
         assert err <= 2e-6, f"d={d}: {err:.3e}"
 
 
+@pytest.mark.parametrize("dtype,d", [(qvp.DTYPE_BF16, 96), (qvp.DTYPE_F16, 96), (qvp.DTYPE_BF16, 256),
+                                     (qvp.DTYPE_F16, 256)])
+def test_infinite_values_stay_infinite_where_weights_are_several_terms(dtype, d):
+    # One infinite value per sequence, in different dims, tiles and parts: the
+    # oracle's whole weights give infinity of its sign in that dim for every head
+    # that reads it and leave the rest finite.
+    print(f"case: infinite values d={d} dtype={dtype}", flush=True)
+    lens = [40, 700, 1500]
+    w = W.custom(lens, 14, 2, d, kv_dtype=dtype, seed=d)
+    image = w.pool_image()
+    elems = image.view(np.uint16).reshape(w.num_pool_blocks, -1)
+    inf = 0x7F80 if dtype == qvp.DTYPE_BF16 else 0x7C00
+    st = w.strides
+    for b, (tok, kv, dim, bits) in enumerate([(33, 0, 5, inf), (600, 1, d - 1, inf | 0x8000), (1499, 0, d // 2, inf)]):
+        frame = w.ids[w.cu_blocks[b] + tok // w.tokens_per_block]
+        at = st["stream_stride"] + tok % w.tokens_per_block * st["token_stride"] + kv * st["head_stride"] + dim
+        elems[frame, at] = bits
+    run = GpuRun(w, image=image)
+    _, ref32 = oracle_decode(w, run.image, run.query)
+    assert np.isinf(ref32).sum() == 3 * 7 and not np.isnan(ref32).any()
+    got = run.decode(out_dtype=qvp.DTYPE_F32)
+    assert np.array_equal(np.where(np.isinf(ref32), ref32, 0), np.where(np.isfinite(got), 0, got))
+    finite = np.isfinite(ref32)
+    assert_close_bf16(np.where(finite, got, 0), np.where(finite, ref32, 0), "the finite dims")
+
+
 def test_decodes_of_one_pack_on_several_streams():
     # Only one stream's decodes may count in the pack's counters: a decode on
     # stream A, then two on B, where the second must not take B's turn as the
