@@ -127,10 +127,11 @@ int qvp_event_elapsed_ms(float* ms, void* start, void* stop);
  * schedule is then cached on the device) with a caller workspace,
  * qvp_append_kv, qvp_copy_blocks, qvp_swap_gather / qvp_swap_scatter,
  * qvp_fill_bytes and device-to-device copies. qvp_pack, qvp_paged_prefill and
- * qvp_mrope_positions upload host-built lists and are not captured. The kernels reset their own merge counters, so a graph may be
- * replayed any number of times; it reads and writes the buffers it was
- * captured with, so a captured decode stays valid until the second qvp_pack
- * after the capture on its batch reuses the packed buffer it reads. */
+ * qvp_mrope_positions upload host-built lists and are not captured. The
+ * kernels reset their own merge counters, so a graph may be replayed any
+ * number of times; it reads and writes the buffers it was captured with, so a
+ * captured decode stays valid until the second qvp_pack after the capture on
+ * its batch reuses the packed buffer it reads. */
 int qvp_graph_begin_capture(void* stream);
 int qvp_graph_end_capture(void* stream, void** graph_exec);
 int qvp_graph_launch(void* graph_exec, void* stream);

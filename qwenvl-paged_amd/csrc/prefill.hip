@@ -10,16 +10,16 @@
 // head r % G at position q_start + r / G; a work item is 128 consecutive rows
 // (a cut may fall inside a position: every wave is full for any group).
 // Its workgroup streams the tokens its last row sees in 32-token tiles: each
-// tile is loaded once, straight into LDS, one tile of compute ahead of its
-// use, into a double buffer holding the K and V rows as in the frame (16-byte
-// chunks XOR-permuted by row so the fragment reads spread over the banks; the
-// PV operands come out of V transposed by ds_read_b64_tr_b16). Each of the
-// four waves holds 32 of the rows in the MFMA columns, a column seeing the
-// tokens up to its position (masks only on tiles that reach the item's first
-// position). The tile loop is
-// software-pipelined over three tiles: PV of tile t - 1 and QK of tile t + 1
-// run beside the softmax of tile t. Items are launched longest context first so the short ones fill the
-// tail.
+// tile is loaded once, straight into LDS, two steps ahead of its use, into a
+// ring of four tiles that hold the K and V rows as in the frame (16-byte chunks
+// XOR-permuted by row so the fragment reads spread over the banks; the PV
+// operands come out of V transposed by ds_read_b64_tr_b16). Each of the four
+// waves holds 32 of the rows in the MFMA columns, a column seeing the tokens up
+// to its position (masks only on tiles that reach the item's first position).
+// The tile loop is software-pipelined over three tiles: PV of tile t - 1 and QK
+// of tile t + 1 run beside the softmax of tile t. Items past 1.25 x a CU's share
+// are cut into pieces that the last one merges (piece_count), and are launched
+// longest first so that the short ones fill the tail.
 //
 // Decode path (any other shape): one virtual sequence per new position (same
 // frames, context p + 1), packed into a private batch and run through
@@ -678,7 +678,8 @@ bool prefill_mfma_supported(const DecodeGeometry& g, uint32_t kv_dtype, uintptr_
     // prefill there. A lane's offset inside a block and the frame stride are
     // kept in 32 bits.
     return (kv_dtype == QVP_DTYPE_BF16 || kv_dtype == QVP_DTYPE_F16) && (g.head_dim == 128 || g.head_dim == 64) &&
-           g.group >= 1 && g.group <= 16 && pow2 && g.tpb >= 16 && aligned && g.token_stride * g.tpb <= 0x7fffffffu && g.block_stride <= 0xffffffffu;
+           g.group >= 1 && g.group <= 16 && pow2 && g.tpb >= 16 && aligned &&
+           g.token_stride * g.tpb <= 0x7fffffffu && g.block_stride <= 0xffffffffu;
 }
 
 template <bool kF16, int kD>
